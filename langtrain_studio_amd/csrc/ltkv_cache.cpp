@@ -143,6 +143,8 @@ struct ltkv_cache {
   // Attention workspace (partition partials), grown on demand.
   uint8_t *ws = nullptr;
   size_t ws_bytes = 0;
+  // States of the parts of small decode launches (ltkv::kPartsBytes).
+  uint8_t *parts = nullptr;
   // The device's static scratch (ltkv_decode_attention_noalloc), looked up at
   // creation; shared by every cache on the device.
   uint8_t *scratch = nullptr;
@@ -1020,6 +1022,8 @@ int ltkv_create(size_t n_layers, size_t kv_dim, size_t n_tokens, int dtype, int 
     if ((e = hipMalloc((void **)&c->d_status, 4 * sizeof(int32_t))) != hipSuccess) rc = hip_fail(e, "hipMalloc(status)");
     else if ((e = hipMemset(c->d_status, 0, 4 * sizeof(int32_t))) != hipSuccess) rc = hip_fail(e, "hipMemset(status)");
   }
+  if (rc == LTKV_OK && (e = hipMalloc((void **)&c->parts, ltkv::kPartsBytes)) != hipSuccess)
+    rc = hip_fail(e, "hipMalloc(parts)");
   const size_t sbytes = c->q8() ? n_layers * c->layer_scales() * 2 : 0;
   if (rc == LTKV_OK && sbytes > 0) {
     if ((e = hipMalloc(&c->ks, sbytes)) != hipSuccess) rc = hip_fail(e, "hipMalloc(K scales)");
@@ -1051,6 +1055,7 @@ void ltkv_destroy(ltkv_cache *c) {
     if (c->d_order_counts) (void)hipFree(c->d_order_counts);
     if (c->d_order_pairs) (void)hipFree(c->d_order_pairs);
     if (c->ws) (void)hipFree(c->ws);
+    if (c->parts) (void)hipFree(c->parts);
     if (c->d_status) (void)hipFree(c->d_status);
     if (c->rope) (void)hipFree(c->rope);
     if (c->plan.done) (void)hipEventDestroy(c->plan.done);
@@ -1462,7 +1467,13 @@ int decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, size
   // Shapes outside the tuned kernels run the generic kernel over whole
   // contexts: no partition partials, so no workspace.
   const bool tuned = ltkv::attention_tuned((int)c->elem, (int)head_dim, (int)group);
-  const ltkv::AttnWorkspace ws =
+  // Small launches run one wave per part of a partition; the parts' states
+  // have a buffer of their own, so neither the workspace nor the scratch is
+  // needed, and the checks below stay those of one wave per partition.
+  const int subs = ltkv::attention_subs((int)c->elem, (int)head_dim, (int)group, (int)(c->kv_dim / head_dim), valu,
+                                        (int64_t)n, (int)max_parts,
+                                        ltkv::max_partition_size((int64_t)max_len, part, split), c->device_count_cu);
+  ltkv::AttnWorkspace ws =
       tuned ? ltkv::attention_workspace((int64_t)n, (int)n_heads, (int)head_dim, (int)max_parts)
             : ltkv::AttnWorkspace{0, 0, 0};
   uint8_t *base = nullptr;
@@ -1473,13 +1484,18 @@ int decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, size
                   "no-allocation scratch",
                   (long long)ws.bytes, ltkv::kScratchBytes);
     base = c->scratch;
-  } else {
+  } else if (subs == 0) {
     if (int rc = ensure_workspace(c, (size_t)ws.bytes)) return rc;
     base = c->ws;
+  }
+  if (subs > 0) {
+    ws = ltkv::attention_workspace((int64_t)n, (int)n_heads, (int)head_dim, (int)max_parts * subs, true);
+    base = c->parts;
   }
   ltkv::AttnArgs a = attn_args(c, layer, n, n_heads, head_dim, scale, d_q, d_out, ws, part,
                                (int)max_parts, base);
   a.split = split;
+  a.subs = subs;
   a.tables = d_tables;
   a.table_stride = (int64_t)table_stride;
   a.rows = d_rows;
@@ -1713,7 +1729,7 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
 
   DeviceGuard dg(c->device);
   if (!dg.ok) return fail(LTKV_ERR_HIP, "hipSetDevice(%d) failed", c->device);
-  const ltkv::AttnWorkspace ws = ltkv::attention_workspace(
+  ltkv::AttnWorkspace ws = ltkv::attention_workspace(
       (int64_t)P.n, (int)P.n_heads, (int)P.head_dim, (int)max_parts, grouped);
   const size_t pre_slots = grouped ? P.n * P.n_heads * (size_t)P.max_pre_parts : 0;
   const size_t pre_o_off = ((size_t)ws.bytes + 255) / 256 * 256;
@@ -1724,6 +1740,17 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
   ltkv::AttnArgs a = attn_args(c, layer, P.n, P.n_heads, P.head_dim, scale, d_q, d_out, ws, part,
                                (int)max_parts, c->ws);
   a.split = split;
+  if (!grouped) {  // a plain decode batch: its small launches as decode_attention's
+    a.subs = ltkv::attention_subs((int)c->elem, (int)P.head_dim, (int)group, a.n_kv_heads, a.valu, a.n,
+                                  (int)max_parts,
+                                  ltkv::max_partition_size((int64_t)(P.sstride * LTKV_BLOCK), part, split),
+                                  c->device_count_cu);
+    if (a.subs > 0) {
+      ws = ltkv::attention_workspace(a.n, a.n_heads, a.head_dim, (int)max_parts * a.subs, true);
+      a.part_o = (float *)(c->parts + ws.part_o_off);
+      a.part_ml = (float *)(c->parts + ws.part_ml_off);
+    }
+  }
   // Short remainders in one partition each and no group-only queries: the
   // decode kernel writes every output itself (folding group partials).
   a.merge_free = grouped && part > 0 && P.max_suffix <= (size_t)(part / split) && !P.empty_with_groups;

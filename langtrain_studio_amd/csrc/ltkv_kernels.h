@@ -112,6 +112,11 @@ struct AttnArgs {
   // (partition_tokens(len) / split tokens each, split 1 or 2); max_parts
   // counts the finer partitions. attention_split gives it for a shape.
   int split;
+  // Parts per partition of a launch with one wave per part (sub_tokens; partial
+  // slots [query][head][max_parts][subs]), or 0: one wave per
+  // partition (slots [query][head][max_parts]). Plain matrix-core decode
+  // only (no group partials); both give the same bits.
+  int subs;
   // Resident block tables: query i reads row rows[i] of `tables` (rows ==
   // nullptr: row i); rows outside [0, n_rows) read row 0.
   const int32_t *rows;
@@ -186,6 +191,27 @@ __host__ __device__ inline int split_partition(int64_t len, int part_tokens, int
   return split == 1 ? pt : (split == 2 ? pt >> 1 : pt / split);
 }
 
+// Tokens per part of a partition in the matrix-core decode kernel.
+// (32 KB of an f16 head's K and V rows up to 8192 tokens of context, more
+// beyond): short enough that one short chat spreads over the chip, and fewer
+// parts where the partitions alone are many, since a wave that streams a
+// whole partition pays ~0.15 us per part for the fold. A function of the
+// query's own length, so its bits do not depend on the batch.
+__host__ __device__ inline int sub_tokens(int64_t len, int head_dim) {
+  const int base = 16384 / head_dim;
+  return len <= 8192 ? base : 2 * base;
+}
+
+// Largest partition (of the matrix-core kernel's cut) of contexts up to
+// max_tokens.
+inline int max_partition_size(int64_t max_tokens, int fixed, int split) {
+  int pt = fixed > 0 ? fixed : partition_tokens(max_tokens, fixed);
+  // the per-query policies grow with the length up to four equal partitions
+  // of the longest such query, then take 1024
+  if (fixed <= 0 && max_tokens > (fixed == kPartCap ? 2048 : 4096)) pt = 1024;
+  return pt / split;
+}
+
 // Upper bound of partitions per query for contexts up to max_tokens (the
 // same for both per-query policies: at most four up to 4096 tokens).
 inline int max_partitions(int64_t max_tokens, int fixed) {
@@ -217,6 +243,13 @@ int attention_split(int elem, int group, int n_kv_heads);
 // The per-query partition policy of a shape (and engine: valu for
 // LTKV_ENGINE_VALU) when none is fixed: kPartCap or 0.
 int attention_part_policy(int elem, int group, int n_kv_heads, bool valu);
+// Parts per partition of a plain decode launch of n queries (AttnArgs::subs),
+// max_parts partitions of at most max_part tokens each; 0: one wave per
+// partition. Their states fit kPartsBytes (a buffer each cache holds from its
+// creation, so no launch allocates for them).
+constexpr size_t kPartsBytes = size_t{32} << 20;
+int attention_subs(int elem, int head_dim, int group, int n_kv_heads, bool valu, int64_t n, int max_parts,
+                   int max_part, int cu_count);
 hipError_t launch_decode_attention(const PoolGeom &g, const AttnArgs &a, hipStream_t s);
 
 // One work-group of shared-prefix attention (mq_attn_kernel): the query rows

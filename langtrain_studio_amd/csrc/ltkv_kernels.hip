@@ -970,6 +970,14 @@ attn_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const floa
   }
 }
 
+// One partial's share (weight a) of a merge: fma, so that every merge kernel
+// gives the same bits.
+__device__ __forceinline__ void merge_add(float a, float l, const f32x4 &po, float &lsum, f32x4 &o) {
+  lsum = __builtin_fmaf(l, a, lsum);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = __builtin_fmaf(po[i], a, o[i]);
+}
+
 // Merge of the context partitions of one (query, head): O = sum_p o_p 2^(m_p-M),
 // L = sum_p l_p 2^(m_p-M), out = O / L. A (query, head) pair takes HD/4
 // threads with 4 output elements each (16-byte loads and stores), a
@@ -1030,8 +1038,7 @@ attn_merge_kernel(const float *__restrict__ part_o, const float *__restrict__ pa
     for (int p = 0; p < NF; ++p) {
       if (p < np) {
         const float a = __builtin_amdgcn_exp2f(m4[p] - mref);
-        lsum += l4[p] * a;
-        o += o4[p] * a;
+        merge_add(a, l4[p], o4[p], lsum, o);
       }
     }
     f32x4 r = {0.f, 0.f, 0.f, 0.f};
@@ -1048,15 +1055,13 @@ attn_merge_kernel(const float *__restrict__ part_o, const float *__restrict__ pa
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int p = 0; p < npre; ++p) {
-    const float a = __builtin_amdgcn_exp2f(pml[2 * p] - mref);
-    lsum += pml[2 * p + 1] * a;
-    o += *reinterpret_cast<const f32x4 *>(pre_o + (qh * max_pre_parts + p) * HD + d) * a;
+    merge_add(__builtin_amdgcn_exp2f(pml[2 * p] - mref), pml[2 * p + 1],
+              *reinterpret_cast<const f32x4 *>(pre_o + (qh * max_pre_parts + p) * HD + d), lsum, o);
   }
 #pragma unroll 4
   for (int p = 0; p < np; ++p) {
-    const float a = __builtin_amdgcn_exp2f(ml[2 * p] - mref);
-    lsum += ml[2 * p + 1] * a;
-    o += *reinterpret_cast<const f32x4 *>(part_o + (qh * max_parts + p) * HD + d) * a;
+    merge_add(__builtin_amdgcn_exp2f(ml[2 * p] - mref), ml[2 * p + 1],
+              *reinterpret_cast<const f32x4 *>(part_o + (qh * max_parts + p) * HD + d), lsum, o);
   }
   f32x4 r = {0.f, 0.f, 0.f, 0.f};
   if (lsum > 0.f) r = f32x4{o.x / lsum, o.y / lsum, o.z / lsum, o.w / lsum};
@@ -1624,7 +1629,179 @@ __device__ __forceinline__ h8 i8x8_to_h8(const u32x2 &w) {
   return h8{p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
 }
 
+// Sum / maximum of a value over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (the
+// four 16-lane rows of the wave), in every lane: v_permlane16_swap and
+// v_permlane32_swap of x with itself give the even and odd rows (the lower
+// and upper halves) in both places, so no exchange goes through LDS.
+template <bool MAX>
+__device__ __forceinline__ float rows_reduce(float x) {
+  auto op = [](float a, float b) { return MAX ? __builtin_fmaxf(a, b) : a + b; };
+  uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  x = op(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  u = __builtin_bit_cast(uint32_t, x);
+  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return op(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
 constexpr float kDecodeSlack = 8.f;  // log2 headroom of the softmax reference
+
+// ----------------------------------------------------------------------------
+// Parts of a partition. The matrix-core decode kernel sums each partition in
+// parts of sub_tokens tokens: every part has its own softmax reference, sum
+// and numerators, and a partition is the left fold of its parts (fold_weights:
+// mul, then fma, in this order everywhere). Whether one wave streams a whole
+// partition and folds the parts in registers, or one wave per part writes its
+// state and the merge folds them, the arithmetic is the same, so a launch may
+// take either by its size alone and a query's bits do not depend on it.
+// ----------------------------------------------------------------------------
+struct FoldWeights {
+  float m, a, b;  // new reference; factors of the running state and of the part
+};
+
+__device__ __forceinline__ FoldWeights fold_weights(float m, float ms) {
+  const float mx = __builtin_fmaxf(m, ms);
+  const bool any = mx != -INFINITY;  // neither side has a score: nothing to rescale
+  return {mx, any ? __builtin_amdgcn_exp2f(m - mx) : 1.f, any ? __builtin_amdgcn_exp2f(ms - mx) : 1.f};
+}
+
+__device__ __forceinline__ float fold_value(const FoldWeights &w, float run, float part) {
+  return __builtin_fmaf(part, w.b, run * w.a);
+}
+
+__device__ __forceinline__ f32x4 fold_value(const FoldWeights &w, const f32x4 &run, const f32x4 &part) {
+  f32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = fold_value(w, run[i], part[i]);
+  return r;
+}
+
+// Merge of a FINE launch: a work-group per (query, head) folds the parts of
+// each partition (a group of HD / 4 threads per partition, 4 output elements
+// a thread, the loads of up to kMergeSubs parts issued together), then merges
+// the partitions as attn_merge_kernel does. The first round's loads are
+// issued before the length is known (indices clamped to the slots the launch
+// has; a part past the query's end is not used, by selection).
+constexpr int kMergeSubs = 8;
+
+template <int HD>
+__global__ void __launch_bounds__(256)
+attn_merge_subs_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml,
+                       const int32_t *__restrict__ lens, float *__restrict__ out, int n_heads, int part_tokens,
+                       int split, int max_parts, int subs, int64_t max_len, const int32_t *__restrict__ qmap) {
+  constexpr int TPP = HD / 4;    // threads per partition
+  constexpr int NG = 256 / TPP;  // partitions per round
+  __shared__ f32x4 so[NG][TPP];
+  __shared__ float sml[NG][2];
+  __shared__ float smx[4];
+  const int64_t pair = blockIdx.x;
+  const int h = (int)(pair % n_heads);
+  const int64_t qx = pair / n_heads;
+  const int64_t qi = qmap ? qmap[qx] : qx;
+  const int64_t qh = qi * n_heads + h;
+  const int g = (int)threadIdx.x / TPP, c = (int)threadIdx.x % TPP;
+  const int64_t slot0 = qh * max_parts * subs;
+  const float *ml = part_ml + 2 * slot0;
+  const float *po = part_o + slot0 * HD + 4 * c;
+  float mr[kMergeSubs], lr[kMergeSubs];
+  f32x4 orr[kMergeSubs];
+  auto load = [&](int p, int s0) {
+    const int pc = p < max_parts ? p : max_parts - 1;
+#pragma unroll
+    for (int u = 0; u < kMergeSubs; ++u) {
+      const int sc = s0 + u < subs ? s0 + u : subs - 1;
+      const int i = pc * subs + sc;
+      mr[u] = ml[2 * i];
+      lr[u] = ml[2 * i + 1];
+      orr[u] = *reinterpret_cast<const f32x4 *>(po + (int64_t)i * HD);
+    }
+  };
+  load(g, 0);
+  int64_t len = lens[qi];
+  if (len < 0) len = 0;
+  if (len > max_len) len = max_len;
+  const int pt = split_partition(len, part_tokens, split);
+  const int np = len > 0 ? div_up_tokens(len, pt) : 1;
+  const int st = sub_tokens(len, HD);
+  // Parts of partition p (an empty query has one, empty, part).
+  auto parts_of = [&](int p) {
+    const int64_t left = len - (int64_t)p * pt;
+    const int tok = left < pt ? (int)left : pt;
+    return tok > 0 ? div_up_tokens(tok, st) : 1;
+  };
+  // The reference of more partitions than one round holds: the maximum of
+  // their parts' references (a partition's is the maximum of its parts').
+  float mx = -INFINITY;
+  if (np > NG) {  // uniform
+    for (int i = (int)threadIdx.x; i < np * subs; i += 256) {
+      const int p = i / subs;
+      if (i - p * subs < parts_of(p)) mx = __builtin_fmaxf(mx, ml[2 * i]);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, off));
+    if ((threadIdx.x & 63) == 0) smx[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    mx = __builtin_fmaxf(__builtin_fmaxf(smx[0], smx[1]), __builtin_fmaxf(smx[2], smx[3]));
+  }
+  float lsum = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < np; p0 += NG) {
+    const int p = p0 + g;
+    if (p0 > 0) load(p, 0);
+    float m = -INFINITY, l = 0.f;
+    f32x4 op = {0.f, 0.f, 0.f, 0.f};
+    if (p < np) {
+      const int ns = parts_of(p);
+      for (int s0 = 0; s0 < ns; s0 += kMergeSubs) {
+        if (s0 > 0) load(p, s0);
+#pragma unroll
+        for (int u = 0; u < kMergeSubs; ++u) {
+          if (s0 + u < ns) {
+            const FoldWeights w = fold_weights(m, mr[u]);
+            m = w.m;
+            l = fold_value(w, l, lr[u]);
+            op = fold_value(w, op, orr[u]);
+          }
+        }
+      }
+    }
+    if (p0 > 0) __syncthreads();  // the last round's readers
+    so[g][c] = op;
+    if (c == 0) {
+      sml[g][0] = m;
+      sml[g][1] = l;
+    }
+    __syncthreads();
+    if (g == 0) {
+      const int cnt = np - p0 < NG ? np - p0 : NG;
+      if (np <= NG)
+        for (int k = 0; k < cnt; ++k) mx = __builtin_fmaxf(mx, sml[k][0]);
+      const float mref = mx == -INFINITY ? 0.f : mx;
+      for (int k = 0; k < cnt; ++k)
+        merge_add(__builtin_amdgcn_exp2f(sml[k][0] - mref), sml[k][1], so[k][c], lsum, o);
+    }
+  }
+  if (g != 0) return;
+  f32x4 r = {0.f, 0.f, 0.f, 0.f};
+  if (np == 1) {  // the decode kernel's own normalisation of a query in one partition
+    const float l1 = sml[0][1];
+    const float inv = 1.f / l1;
+    if (l1 > 0.f) r = so[0][c] * inv;
+  } else if (lsum > 0.f) {
+    r = f32x4{o.x / lsum, o.y / lsum, o.z / lsum, o.w / lsum};
+  }
+  *reinterpret_cast<f32x4 *>(out + qh * HD + 4 * c) = r;
+}
+
+// Launch check of a FINE launch, then its merge.
+template <int HD>
+hipError_t launch_merge_subs(const AttnArgs &a, hipStream_t s) {
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  attn_merge_subs_kernel<HD><<<(unsigned)(a.n * a.n_heads), 256, 0, s>>>(
+      a.part_o, a.part_ml, a.lens, a.out, a.n_heads, a.part_tokens, a.split, a.max_parts, a.subs, a.max_len, a.qmap);
+  return hipGetLastError();
+}
 
 // The matrix-core products take Q as f16 operands. A query head whose scaled
 // Q (x = q * scale * log2 e) reaches the f16 range (|x| >= 65504) enters them
@@ -1671,6 +1848,19 @@ __device__ __forceinline__ int order_class(int tokens, int k) {
   return c < kOrderClasses - 1 ? c : kOrderClasses - 1;
 }
 
+// Inclusive prefix sum over the 64 lanes (DPP row shifts within each row of
+// 16, then the rows' totals broadcast into the rows after them): ~10 vector
+// instructions where shuffles took a round trip through LDS per step.
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
 // Query q's length (clamped), partition size and partition count.
 __device__ __forceinline__ void decode_query_parts(const int32_t *__restrict__ lens, int64_t q, int64_t max_len,
                                                    int part_tokens, int split, int &clen, int &pt, int &np) {
@@ -1712,15 +1902,39 @@ __device__ __forceinline__ int decode_order_setup(const int32_t *__restrict__ le
       decode_query_parts(lens, (int64_t)c * 64 + lane, max_len, part_tokens, split, sh.len[c], pt[c],
                          sh.items[c]);
   }
-  if constexpr (RUNS) {  // the run length from the batch's partition items (a wave-wide sum)
-    int total = 0;
+  if constexpr (RUNS) {
+    // The run length: the shortest whose items all start at once (they then
+    // end together), or, with more items than that, the one whose items fill
+    // the rounds of the wave slots best (longer runs on a tie: fewer starts).
+    // A remainder under an eighth of a partition is not counted as an item.
+    // Runs of partitions / slots left a nearly empty round: 24 queries of
+    // 32769 tokens are 1056 runs of three on 1024 slots, and the last 32 ran
+    // alone (614 us; 518 us with single partitions; 476 us with runs of four).
+    int np[kOrderChunks], total[4];
 #pragma unroll
-    for (int c = 0; c < kOrderChunks; ++c) total += sh.items[c];
+    for (int c = 0; c < kOrderChunks; ++c) {
+      const int rest = (int)((uint32_t)sh.len[c] % (uint32_t)pt[c]);
+      np[c] = rest > 0 && rest < pt[c] >> 3 && sh.items[c] > 1 ? sh.items[c] - 1 : sh.items[c];
+    }
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) total += __shfl_xor(total, off);
-    const int64_t waves = (int64_t)__builtin_amdgcn_readfirstlane(total) * n_groups;
-    k = slots > 0 && waves >= 2 * (int64_t)slots ? (int)(waves / slots) : 1;
-    k = k < max_run ? k : max_run;
+    for (int r = 0; r < 4; ++r) {
+      total[r] = 0;
+#pragma unroll
+      for (int c = 0; c < kOrderChunks; ++c) total[r] += (int)((uint32_t)(np[c] + r) / (uint32_t)(r + 1));
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) total[r] = __builtin_amdgcn_readlane(wave_scan(total[r]), 63);
+    int64_t best = 0;
+#pragma unroll
+    for (int r = 1; r <= 4; ++r) {
+      const uint32_t items = (uint32_t)total[r - 1] * (uint32_t)n_groups;
+      const int64_t rounds = (items + (uint32_t)slots - 1) / (uint32_t)slots;
+      const int64_t time = rounds <= 1 ? 0 : rounds * r;
+      if (r == 1 || (r <= max_run && (time < best || (time == best && time > 0)))) {
+        best = time;
+        k = r;
+      }
+    }
   } else {
     (void)n_groups;
     (void)slots;
@@ -1752,18 +1966,14 @@ __device__ __forceinline__ int decode_order_setup(const int32_t *__restrict__ le
 // stay in scalar registers.
 __device__ __forceinline__ bool decode_order_find(int64_t t, int64_t n, int lane, const int32_t *hist,
                                                   const OrderShapes &sh, int64_t &qx, int &part, int &qlen) {
-  int cls = -1;
-  int64_t base = 0;
-  for (int k = kOrderClasses - 1; k >= 0; --k) {
-    const int c = __builtin_amdgcn_readfirstlane(hist[k]);
-    if (t < base + c) {
-      cls = k;
-      break;
-    }
-    base += c;
-  }
-  if (cls < 0) return false;
-  t -= base;
+  // the class that holds item t, classes in descending order
+  const int count = lane < kOrderClasses ? hist[kOrderClasses - 1 - lane] : 0;
+  const int upto = wave_scan(count);
+  const uint64_t in = __builtin_amdgcn_ballot_w64((int64_t)upto > t);
+  if (!in) return false;
+  const int first = __builtin_ctzll(in);
+  const int cls = kOrderClasses - 1 - first;
+  t -= __builtin_amdgcn_readlane(upto, first) - __builtin_amdgcn_readlane(count, first);
 #pragma unroll
   for (int c = 0; c < kOrderChunks; ++c) {
     const int64_t c0 = (int64_t)c * 64;
@@ -1771,21 +1981,16 @@ __device__ __forceinline__ bool decode_order_find(int64_t t, int64_t n, int lane
     // this class's items of the lane's query: its full partitions (parts
     // 0 .. items - 2) and / or its last one (part items - 1)
     const int v = (sh.key[c] == cls ? sh.items[c] - 1 : 0) + (sh.keyl[c] == cls ? 1 : 0);
-    int incl = v;  // inclusive prefix sum over the wave
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int y = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += y;
-    }
-    const int tot = __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
+    const int incl = wave_scan(v);
+    const int tot = __builtin_amdgcn_readlane(incl, 63);
     if (t < tot) {
       const uint64_t hit = __builtin_amdgcn_ballot_w64(incl > t);
       const int j = __builtin_ctzll(hit);
-      const int end = __builtin_amdgcn_readfirstlane(__shfl(incl, j, 64));
-      const int cnt = __builtin_amdgcn_readfirstlane(__shfl(v, j, 64));
-      const int key = __builtin_amdgcn_readfirstlane(__shfl(sh.key[c], j, 64));
-      const int items = __builtin_amdgcn_readfirstlane(__shfl(sh.items[c], j, 64));
-      qlen = __builtin_amdgcn_readfirstlane(__shfl(sh.len[c], j, 64));
+      const int end = __builtin_amdgcn_readlane(incl, j);
+      const int cnt = __builtin_amdgcn_readlane(v, j);
+      const int key = __builtin_amdgcn_readlane(sh.key[c], j);
+      const int items = __builtin_amdgcn_readlane(sh.items[c], j);
+      qlen = __builtin_amdgcn_readlane(sh.len[c], j);
       qx = c0 + j;
       part = key == cls ? (int)(t - (end - cnt)) : items - 1;
       return true;
@@ -1853,8 +2058,14 @@ __device__ __forceinline__ h8 i8x8_to_h8_biased(const u32x2 &w) {
 // vector value or a 64-bit division it cost SGPR spills and 10%.
 constexpr int kDecodeWaves = 4;
 
-template <typename T, int HD, int G, int NH, bool RUNS>
-__global__ void __launch_bounds__(64 * kDecodeWaves)
+// FINE: one wave (a work-group of its own) per part of a partition, in
+// query order, its state written for attn_merge_subs_kernel. For launches
+// whose partitions would leave most of the chip idle: a wave streams a
+// 16-token tile of a Llama-3-8B pair of heads (16 KB) in ~1.1 us and one CU
+// takes in ~56 GB/s at most, so a partition of 1024 tokens lasts ~75 us
+// however idle the chip is, and four waves of one CU share that rate.
+template <typename T, int HD, int G, int NH, bool RUNS, bool FINE>
+__global__ void __launch_bounds__(64 * kDecodeWaves, NH == 1 && HD == 64 ? 4 : 1)
 attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const float *__restrict__ q,
                  const int32_t *__restrict__ tables, int64_t table_stride,
                  const int32_t *__restrict__ lens, float *__restrict__ out, float *__restrict__ part_o,
@@ -1866,8 +2077,9 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
                  int64_t max_len, const float *__restrict__ pre_o, const float *__restrict__ pre_ml,
                  int max_pre_parts, const int32_t *__restrict__ new_slots,
                  const float *__restrict__ new_k, const float *__restrict__ new_v, int64_t new_stride,
-                 T *kdst, T *vdst, int64_t n_queries, int order, int slots, int pair_items,
+                 T *kdst, T *vdst, int64_t n_queries, int order, int slots, int pair_items, int subs,
                  int32_t *__restrict__ status) {
+  static_assert(!(RUNS && FINE), "runs of partitions, or parts of one");
 #ifdef LTKV_TIMELINE
   unsigned long long tl_[8] = {__builtin_amdgcn_s_memrealtime(), 0, 0, 0, 0, 0, 0, 0};
 #endif
@@ -1900,7 +2112,9 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   constexpr int VPITCH = HD * 2 + (!Q8 && HD == 128 ? 32 : 16);
   constexpr int NQ = NH * G;               // query heads of the wave
   constexpr int NSC = NH * KS * 16;        // q8_0 scale entries of a tile, K or V
-  constexpr int STAGES = NH == 2 && Q8 ? 2 : 3;  // tiles in flight + 1
+    // tiles in flight + 1 (FINE f16 pairs: two waves a SIMD with two, one with
+  // three: 16.1 against 14.4 us for one Llama-3-8B query of 5003 tokens)
+  constexpr int STAGES = NH == 2 && (Q8 || (FINE && HD == 128)) ? 2 : 3;  // tiles in flight + 1
   using KV = typename BufVec<KB>::type;
   using SV = uint32_t;  // one or two b16 scale entries
   static_assert(NQ <= 8, "hi and lo columns of the wave's query heads must fit 16");
@@ -1928,9 +2142,10 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   // take the kernel without it (RUNS false): kernels at two waves per SIMD
   // (q8_0, one-head waves) lost their occupancy or 3% with it.
   static_assert(!RUNS || (NH == 2 && !Q8), "runs of partitions: f16 two-head waves");
-  constexpr int kRunSlots = RUNS ? 3 : 1;
-  __shared__ __attribute__((aligned(16))) f32x4 srun_o[NW][kRunSlots][RUNS ? DT : 1][RUNS ? NQ * 4 : 1];
-  __shared__ float srun_ml[NW][kRunSlots][RUNS ? NQ : 1][2];
+  constexpr int kRunSlots = RUNS ? 3 : 0;
+  // ... and one slot more for the partition whose parts are being folded
+  __shared__ __attribute__((aligned(16))) f32x4 srun_o[FINE ? 1 : NW][kRunSlots + 1][FINE ? 1 : DT][FINE ? 1 : NQ * 4];
+  __shared__ float srun_ml[RUNS ? NW : 1][RUNS ? kRunSlots : 1][RUNS ? NQ : 1][2];
 
   __shared__ int32_t shist[kOrderClasses];
 
@@ -1939,7 +2154,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   // query w / max_parts; with `order`, item w of the longest-first list
   // (decode_order_find), a run of `run` consecutive partitions of a query.
   const int n_groups = n_kv_heads / NH;
-  const unsigned gw = blockIdx.x * NW + wv;  // the grid's wave (the launch keeps it below 2^32)
+  const unsigned gw = blockIdx.x * (FINE ? blockDim.x >> 6 : NW) + wv;  // the grid's wave (the launch keeps it below 2^32)
   const int kvh0 = (int)(gw % n_groups) * NH;
   const int lane = threadIdx.x & 63;
   const int lr = lane & 15, lq = lane >> 4;
@@ -1959,7 +2174,8 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   }
   OrderShapes osh;
   int run = 1;
-  if (order)
+  int sub = 0;  // FINE: the wave's part of its partition
+  if (!FINE && order)
     run = decode_order_setup<(NW > 1), RUNS>(lens, n_queries, max_len, part_tokens, split, lane, shist, osh,
                                              n_groups, slots, kRunSlots + 1);
 
@@ -1998,8 +2214,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         amax = __builtin_fmaxf(amax, __builtin_fabsf((e < 4 ? qr[2 * ks][e] : qr[2 * ks + 1][e - 4]) * qscale));
-    amax = __builtin_fmaxf(amax, __shfl_xor(amax, 16));
-    amax = __builtin_fmaxf(amax, __shfl_xor(amax, 32));
+    amax = rows_reduce<true>(amax);
     const int qex = q_range_exp(amax);
     const float qinv = __builtin_ldexpf(1.f, -qex);
     qmul = __builtin_ldexpf(1.f, qex);
@@ -2023,9 +2238,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
         for (int a = 0; a < NH; ++a)
 #pragma unroll
           for (int e = 0; e < 8; ++e) t += (float)qb[a][ks][e];
-        t += __shfl_xor(t, 16);
-        t += __shfl_xor(t, 32);
-        qbias[ks] = 1152.f * t;
+        qbias[ks] = 1152.f * rows_reduce<false>(t);
       }
     }
   };
@@ -2086,20 +2299,21 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
     it.valid = false;
     int64_t qx;
     int part, olen = 0;
-    if (order) {
+    if (!FINE && order) {
       if (!decode_order_find(wave_idx, n_queries, lane, shist, osh, qx, part, olen)) return;
       // uniform over the wave: keep them (and the table and buffer addresses
       // derived from them) in scalar registers
       qx = __builtin_amdgcn_readfirstlane((int)qx);
       part = __builtin_amdgcn_readfirstlane(part);
     } else {
-      part = (int)(wave_idx % max_parts);
-      qx = wave_idx / max_parts;
-      if (NW > 1 && qx >= n_queries) return;  // waves past the grid's last item
+      const uint32_t per_query = (uint32_t)max_parts * (FINE ? (uint32_t)subs : 1u);
+      part = (int)((uint32_t)wave_idx % per_query);
+      qx = (uint32_t)wave_idx / per_query;
+      if (!FINE && qx >= n_queries) return;  // waves past the grid's last item
     }
     const int64_t qi = qmap ? qmap[qx] : qx;
     int64_t len;
-    if (order) {
+    if (!FINE && order) {
       len = olen;  // the order scan read and clamped it (ordered launches have no query map)
     } else {
       len = lens[qi];
@@ -2111,11 +2325,28 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
     if (pre_parts && (pre_parts[qi] < 0 || (pre_parts[qi] > 0 && len == 0))) return;
     const int pt = split_partition(len, part_tokens, split);
     const int np = len > 0 ? div_up_tokens(len, pt) : 1;
+    if constexpr (FINE) {
+      // The query's parts come first in its index range, partition by
+      // partition, so the waves past them are the range's end (with a fixed
+      // number of waves per partition, the waves of parts that long contexts
+      // do not have fell on the same XCDs: one query of 32000 tokens 45.8
+      // us, 38 us so).
+      const int per_part = div_up_tokens(pt, sub_tokens(len, HD));
+      const int p = (int)((uint32_t)part / (uint32_t)per_part);
+      sub = part - p * per_part;
+      part = p;
+    }
     // the item's partitions: run of them from part * run (run 1 without order)
     part *= run;
     if (part >= np) return;
     const int plast = part + run - 1 < np - 1 ? part + run - 1 : np - 1;
-    const int64_t tok0 = (int64_t)part * pt, tend = (int64_t)(plast + 1) * pt;
+    int64_t tok0 = (int64_t)part * pt, tend = (int64_t)(plast + 1) * pt;
+    if constexpr (FINE) {  // the wave's part; parts past the partition or the context hold nothing
+      const int st = sub_tokens(len, HD);
+      tok0 += (int64_t)sub * st;
+      if (sub > 0 && (tok0 >= tend || tok0 >= len)) return;
+      tend = tend < tok0 + st ? tend : tok0 + st;
+    }
     it.qi = qi;
     it.len = len;
     it.part = part;
@@ -2151,7 +2382,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
     it.cell = -1;
     kr[0] = kr[1] = vr[0] = vr[1] = f32x4{0.f, 0.f, 0.f, 0.f};
     if constexpr (!Q8) {
-      if (new_slots && plast == np - 1 && len > 0) {  // uniform
+      if (new_slots && it.tok1 == len && len > 0) {  // uniform
         const int32_t cell = scalar_read(new_slots, qi);
         // The cell must be position len - 1 of the query's table (what the
         // claim returned for it); otherwise write-then-attend would differ.
@@ -2336,18 +2567,20 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
     const float lmax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(sc[0], sc[1]),
                                                      __builtin_elementwise_maximum(sc[2], sc[3]));
     if (__builtin_amdgcn_ballot_w64(lmax > m_thr)) {
-      float mx = __builtin_fmaxf(lmax, __shfl_xor(lmax, 16));
-      mx = __builtin_fmaxf(mx, __shfl_xor(mx, 32));
+      const float mx = rows_reduce<true>(lmax);
       if (mx > m_thr) {
         const float alpha = __builtin_amdgcn_exp2f(m_ref - mx);
+        const bool held = m_ref != -INFINITY;  // else the column's accumulators are still empty
         m_ref = mx;
         m_thr = mx + kDecodeSlack;
         m_off = mx;
-        l_run *= alpha;
+        if (__builtin_amdgcn_ballot_w64(held)) {
+          l_run *= alpha;
 #pragma unroll
-        for (int a = 0; a < OS; ++a)
+          for (int a = 0; a < OS; ++a)
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt) oacc[a][dt] *= alpha;
+            for (int dt = 0; dt < DT; ++dt) oacc[a][dt] *= alpha;
+        }
       }
     }
     float p[4];
@@ -2392,18 +2625,45 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
         for (int dt = 0; dt < DT; ++dt) oacc[0][dt] = a == my_head ? oacc[a][dt] : oacc[0][dt];
     }
     // Column sums over the four lane rows; hi + lo parts of the numerators.
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
+    l_run = rows_reduce<false>(l_run);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) oacc[0][dt][i] += dpp<0x140>(oacc[0][dt][i]);
   };
-  // Partial (numerators, reference, sum) of partition it.part, after reduce_acc.
+  // The fold of a partition's parts so far, between two of its parts: the
+  // numerators in the wave's LDS slot (registers would cost the q8_0 and
+  // one-head kernels their second or third wave per SIMD), reference and sum
+  // in registers.
+  float mrun = -INFINITY, lrun = 0.f;
+  bool has_run = false;  // the partition has earlier parts (uniform)
+  auto run_slot = [&]() __attribute__((always_inline)) { return RUNS ? cur.part - cur.p0 : 0; };
+  // The part that ends, folded into the partition: the state after it in
+  // oacc[0], m_ref and l_run. (FINE: the part's own state.)
+  auto fold_part = [&]() __attribute__((always_inline)) {
+    reduce_acc();
+    if constexpr (!FINE) {
+      if (has_run) {
+        const FoldWeights w = fold_weights(mrun, m_ref);
+        m_ref = w.m;
+        l_run = fold_value(w, lrun, l_run);
+        if (hi_lane) {
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt)
+            oacc[0][dt] = fold_value(w, srun_o[wv][run_slot()][dt][lq * NQ + lr], oacc[0][dt]);
+        }
+      } else {  // the fold of one part: a zero state
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) oacc[0][dt] += 0.f;
+      }
+    }
+  };
+  // Partial (numerators, reference, sum) of partition it.part, or of the
+  // wave's part of it.
   auto write_partial = [&](const Item &it) __attribute__((always_inline)) {
     if (!hi_lane) return;
     const int64_t qh = it.qi * n_heads + (int64_t)kvh0 * G + lr;
-    const int64_t pi = qh * max_parts + it.part;
+    const int64_t pi = FINE ? (qh * max_parts + it.part) * subs + sub : qh * max_parts + it.part;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
       *reinterpret_cast<f32x4 *>(part_o + pi * HD + 16 * dt + 4 * lq) = oacc[0][dt];
@@ -2416,7 +2676,11 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   // The item's result: the output (one partition) or the partial of its last
   // partition.
   auto finish = [&](const Item &it) __attribute__((always_inline)) {
-    reduce_acc();
+    fold_part();
+    if constexpr (FINE) {
+      write_partial(it);
+      return;
+    }
     if (!hi_lane) return;  // lane (j, lq) holds rows d = 16 dt + 4 lq + i of the wave's query head j
     if (it.np > 1) {
       write_partial(it);
@@ -2499,45 +2763,59 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
     else if (left > 24) __builtin_amdgcn_s_setprio(1);
     else __builtin_amdgcn_s_setprio(0);
   };
-  // The tile loop stops at `stop`: the item's end or, inside a run, the end
-  // of the current partition. There the partition's partial goes to the
-  // wave's LDS slot cur.part - cur.p0 (fewer than kRunSlots: runs are at
-  // most kRunSlots + 1 partitions) and the next partition starts from empty
-  // accumulators (the tiles in flight are the next partition's). One test
-  // per tile, as for the item's end alone: a separate test per tile cost the
-  // Qwen2.5-7B step 3% (the tiles' work no longer overlapped across it).
-  auto part_stop = [&]() __attribute__((always_inline)) {
+  // The tile loop stops at `stop`: the item's end or the end of a part, where
+  // the part's state is folded into the partition's (the tiles in flight are
+  // the next part's). At a partition's end inside a run, the partition's
+  // state goes to the wave's LDS slot cur.part - cur.p0 (fewer than
+  // kRunSlots: runs are at most kRunSlots + 1 partitions). One test per tile:
+  // a separate test for the partition's end cost the Qwen2.5-7B step 3% (the
+  // tiles' work no longer overlapped across it).
+  auto part_end = [&]() __attribute__((always_inline)) {
     const int e = (cur.part + 1) * cur.pt_tiles;
     return e < cur.b1 ? e : cur.b1;
   };
-  int stop = part_stop();
+  int pstop = part_end();
+  const int sub_tiles = sub_tokens(cur.len, HD) >> 4;
+  auto sub_end = [&](int from) __attribute__((always_inline)) {
+    return from + sub_tiles < pstop ? from + sub_tiles : pstop;
+  };
+  int stop = FINE ? cur.b1 : sub_end(b);
   auto next_part = [&]() __attribute__((always_inline)) {
-    if constexpr (RUNS) {
-      reduce_acc();
-      const int slot = cur.part - cur.p0;
+    if constexpr (!FINE) {
+      fold_part();
+      const int slot = run_slot();
       if (hi_lane) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) srun_o[wv][slot][dt][lq * NQ + lr] = oacc[0][dt];
-        if (lq == 0) {
-          srun_ml[wv][slot][lr][0] = m_ref;
-          srun_ml[wv][slot][lr][1] = l_run;
+      }
+      mrun = m_ref;
+      lrun = l_run;
+      has_run = true;
+      if constexpr (RUNS) {
+        if (b >= pstop) {  // the partition's end
+          if (hi_lane && lq == 0) {
+            srun_ml[wv][slot][lr][0] = m_ref;
+            srun_ml[wv][slot][lr][1] = l_run;
+          }
+          has_run = false;
+          ++cur.part;
+          pstop = part_end();
         }
       }
       reset();
-      ++cur.part;
-      stop = part_stop();
+      stop = sub_end(b);
     }
   };
   // After tile b - 1 (b incremented): false when the item is done.
   auto more = [&]() __attribute__((always_inline)) {
-    if constexpr (RUNS) {
+    if constexpr (FINE) {
+      return b < cur.b1;
+    } else {
       if (b >= stop) {
         if (b >= cur.b1) return false;
         next_part();
       }
       return true;
-    } else {
-      return b < cur.b1;
     }
   };
   if (b < cur.b1) {
@@ -2630,18 +2908,23 @@ inline bool decode_ordered(const AttnArgs &a) {
 // One wave per item (a partition of NH kv heads of one query), kDecodeWaves
 // consecutive items per work-group; the grid is rounded up to whole
 // work-groups and the waves past the last item leave at once.
-template <typename T, int HD, int G, int NH, bool RUNS>
+template <typename T, int HD, int G, int NH, bool RUNS, bool FINE = false>
 hipError_t launch_attn_mfma_k(const PoolGeom &g, const AttnArgs &a, int slots, int pair_items, hipStream_t s) {
-  constexpr int nw = kDecodeWaves;
-  const unsigned grid = (unsigned)((a.n * (a.n_kv_heads / NH) * a.max_parts + nw - 1) / nw);
-  attn_mfma_kernel<T, HD, G, NH, RUNS><<<grid, 64 * nw, 0, s>>>(
+  const int64_t waves = a.n * (a.n_kv_heads / NH) * a.max_parts * (FINE ? a.subs : 1);
+  // FINE work-groups of one wave up to four a CU, so that few waves spread
+  // over the CUs (one Llama-3-8B query of 5003 tokens: 14.4 us against 17.5
+  // with four waves a work-group); beyond, fewer work-groups to dispatch.
+  const int nw = FINE && waves <= 4 * (int64_t)a.cu_count ? 1 : kDecodeWaves;
+  const unsigned grid = (unsigned)((waves + nw - 1) / nw);
+  attn_mfma_kernel<T, HD, G, NH, RUNS, FINE><<<grid, 64 * nw, 0, s>>>(
       static_cast<const T *>(a.k_layer), static_cast<const T *>(a.v_layer), a.q, a.tables, a.table_stride,
       a.lens, a.out, a.part_o, a.part_ml, a.n_kv_heads, g.n_blocks, g.block_stride, g.slot_stride,
       g.head_stride, a.scale * kLog2e, a.part_tokens, a.split, a.max_parts, a.pre_parts, a.qmap,
       static_cast<const uint16_t *>(a.k_scale), static_cast<const uint16_t *>(a.v_scale), a.rows, a.n_rows,
       a.max_len, a.pre_o, a.pre_ml, a.max_pre_parts, a.new_slots, a.new_k, a.new_v, a.new_stride,
       static_cast<T *>(const_cast<void *>(a.k_layer)), static_cast<T *>(const_cast<void *>(a.v_layer)), a.n,
-      decode_ordered(a) ? 1 : 0, slots, pair_items, a.status);
+      decode_ordered(a) ? 1 : 0, slots, pair_items, a.subs, a.status);
+  if constexpr (FINE) return launch_merge_subs<HD>(a, s);
   return launch_merge<HD>(a, s, true);
 }
 
@@ -2652,12 +2935,13 @@ hipError_t launch_attn_mfma_k(const PoolGeom &g, const AttnArgs &a, int slots, i
 template <typename T, int HD, int G, int NH>
 hipError_t launch_attn_mfma_t(const PoolGeom &g, const AttnArgs &a, hipStream_t s) {
   constexpr int nw = kDecodeWaves;
+  if (a.subs > 0) return launch_attn_mfma_k<T, HD, G, NH, false, true>(g, a, 0, 0, s);
   if constexpr (NH == 2 && !std::is_same_v<T, int8_t>) {
     // Waves the chip holds at once (work-groups per CU from the kernel's
     // registers and LDS).
     static const int per_cu = [] {
       int blocks = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, attn_mfma_kernel<T, HD, G, NH, true>, 64 * nw,
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, attn_mfma_kernel<T, HD, G, NH, true, false>, 64 * nw,
                                                        0) != hipSuccess)
         blocks = 0;
       return blocks * nw;
@@ -2670,7 +2954,7 @@ hipError_t launch_attn_mfma_t(const PoolGeom &g, const AttnArgs &a, hipStream_t 
   // the work-groups the chip starts with are paired longest with shortest.
   static const int wg_per_cu = [] {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, attn_mfma_kernel<T, HD, G, NH, false>, 64 * nw, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, attn_mfma_kernel<T, HD, G, NH, false, false>, 64 * nw, 0) !=
         hipSuccess)
       blocks = 0;
     return blocks;
@@ -3894,6 +4178,29 @@ int attention_part_policy(int elem, int group, int n_kv_heads, bool valu) {
   (void)group;
   (void)n_kv_heads;
   return !valu && elem == 2 ? kPartCap : 0;
+}
+
+int attention_subs(int elem, int head_dim, int group, int n_kv_heads, bool valu, int64_t n, int max_parts,
+                   int max_part, int cu_count) {
+  if (elem == 4 || valu || !attention_tuned(elem, head_dim, group)) return 0;
+  const bool pairs = group <= 4 && n_kv_heads % 2 == 0;  // two kv heads a wave
+  const int64_t waves = n * (n_kv_heads / (pairs ? 2 : 1)) * max_parts;
+  const int64_t subs = div_up_tokens(max_part, sub_tokens(0, head_dim));
+  // Where the partitions number at most half the SIMDs. Measured (us,
+  // partitions against parts; Llama-3-8B f16): 16 queries of 200-3000 tokens
+  // 80.5 / 32.2, 32 of 2048-4096 (512 partitions) 92-103 / 82; 64 of them
+  // (1024) 129 / 161. head_dim 64 partitions take half the time (TinyLlama,
+  // 256: 36 / 25; 512: 41 / 46), q8_0 waves of one head nearly as long as
+  // f16 ones at half the bytes (Qwen2.5-7B, 512: 69 / 42; 1024: 72 / 69).
+  // Partitions of up to three parts gain only from the work-groups of one
+  // wave, up to one a CU (Qwen2.5-7B q8_0, 1024 of 192 tokens: 26.3 / 27.7).
+  int64_t limit = 2 * (int64_t)cu_count;
+  if (subs < 4) limit = cu_count;
+  else if (head_dim == 64) limit = 3 * (int64_t)cu_count / 2;
+  else if (elem == 1 && !pairs) limit = 4 * (int64_t)cu_count;
+  if (waves > limit) return 0;
+  const int64_t bytes = n * n_kv_heads * group * max_parts * subs * (head_dim + 2) * 4;
+  return bytes > (int64_t)kPartsBytes ? 0 : (int)subs;
 }
 
 int mq_rows(int, int) { return 32 * kMqWaves; }
