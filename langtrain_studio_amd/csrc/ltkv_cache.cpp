@@ -143,7 +143,8 @@ struct ltkv_cache {
   // Attention workspace (partition partials), grown on demand.
   uint8_t *ws = nullptr;
   size_t ws_bytes = 0;
-  // States of the parts of small decode launches (ltkv::kPartsBytes).
+  // Partials of small launches (ltkv::kPartsBytes, held from creation): the
+  // states of parts, and partition partials of up to half its size.
   uint8_t *parts = nullptr;
   // The device's static scratch (ltkv_decode_attention_noalloc), looked up at
   // creation; shared by every cache on the device.
@@ -421,6 +422,19 @@ int ensure_workspace(ltkv_cache *c, size_t bytes) {
   return LTKV_OK;
 }
 
+// Memory for a launch's partials: the buffer held from the cache's creation
+// for up to half of it (no allocation on a first call; the launches of a
+// cache follow each other on its stream), the workspace beyond.
+int workspace(ltkv_cache *c, size_t bytes, uint8_t **base) {
+  if (bytes <= ltkv::kPartsBytes / 2) {
+    *base = c->parts;
+    return LTKV_OK;
+  }
+  if (int rc = ensure_workspace(c, bytes)) return rc;
+  *base = c->ws;
+  return LTKV_OK;
+}
+
 // Uploads the resident-table changes made since the last call: only the
 // changed entries of changed rows, as (row, col, value) triples through
 // pinned staging, applied by one small kernel on the cache stream. Growing
@@ -560,6 +574,15 @@ ltkv::AttnArgs attn_args(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, 
   a.status = c->d_status;
   a.cu_count = c->device_count_cu;
   return a;
+}
+
+// The part states of attn_wide_kernel's shapes go to the cache's parts buffer.
+void set_wide_parts(const ltkv_cache *c, ltkv::AttnArgs &a, size_t group, size_t max_len) {
+  if (!ltkv::attention_wide((int)c->elem, a.head_dim, (int)group, a.valu)) return;
+  a.wide_parts = ltkv::attention_wide_parts(a.n, a.n_heads, a.head_dim, (int64_t)max_len);
+  const ltkv::AttnWorkspace ws = ltkv::attention_workspace(a.n, a.n_heads, a.head_dim, a.wide_parts, true);
+  a.part_o = (float *)(c->parts + ws.part_o_off);
+  a.part_ml = (float *)(c->parts + ws.part_ml_off);
 }
 
 // Fewest shared full blocks and members for a prefix group.
@@ -1485,8 +1508,7 @@ int decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, size
                   (long long)ws.bytes, ltkv::kScratchBytes);
     base = c->scratch;
   } else if (subs == 0) {
-    if (int rc = ensure_workspace(c, (size_t)ws.bytes)) return rc;
-    base = c->ws;
+    if (int rc = workspace(c, (size_t)ws.bytes, &base)) return rc;
   }
   if (subs > 0) {
     ws = ltkv::attention_workspace((int64_t)n, (int)n_heads, (int)head_dim, (int)max_parts * subs, true);
@@ -1496,6 +1518,7 @@ int decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, size
                                (int)max_parts, base);
   a.split = split;
   a.subs = subs;
+  set_wide_parts(c, a, group, max_len);
   a.tables = d_tables;
   a.table_stride = (int64_t)table_stride;
   a.rows = d_rows;
@@ -1734,12 +1757,14 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
   const size_t pre_slots = grouped ? P.n * P.n_heads * (size_t)P.max_pre_parts : 0;
   const size_t pre_o_off = ((size_t)ws.bytes + 255) / 256 * 256;
   const size_t pre_ml_off = pre_o_off + pre_slots * P.head_dim * 4;
-  if (int rc = ensure_workspace(c, pre_ml_off + pre_slots * 2 * 4)) return rc;
+  uint8_t *base = nullptr;
+  if (int rc = workspace(c, pre_ml_off + pre_slots * 2 * 4, &base)) return rc;
   const int32_t *d = reinterpret_cast<const int32_t *>(P.d);
   const ltkv::PoolGeom g = head_geom(c, P.head_dim);
   ltkv::AttnArgs a = attn_args(c, layer, P.n, P.n_heads, P.head_dim, scale, d_q, d_out, ws, part,
-                               (int)max_parts, c->ws);
+                               (int)max_parts, base);
   a.split = split;
+  set_wide_parts(c, a, group, P.sstride * LTKV_BLOCK);
   if (!grouped) {  // a plain decode batch: its small launches as decode_attention's
     a.subs = ltkv::attention_subs((int)c->elem, (int)P.head_dim, (int)group, a.n_kv_heads, a.valu, a.n,
                                   (int)max_parts,
@@ -1765,8 +1790,8 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
   }
   if (grouped) {
     a.pre_parts = d + P.off_pre;
-    a.pre_o = (float *)(c->ws + pre_o_off);
-    a.pre_ml = (float *)(c->ws + pre_ml_off);
+    a.pre_o = (float *)(base + pre_o_off);
+    a.pre_ml = (float *)(base + pre_ml_off);
     a.max_pre_parts = P.max_pre_parts;
     ltkv::MqArgs m{};
     m.k_layer = a.k_layer;

@@ -117,6 +117,9 @@ struct AttnArgs {
   // partition (slots [query][head][max_parts]). Plain matrix-core decode
   // only (no group partials); both give the same bits.
   int subs;
+  // Parts per query of attn_wide_kernel (partial slots [query][head][parts]),
+  // or 0: each work-group folds its query's whole context itself.
+  int wide_parts;
   // Resident block tables: query i reads row rows[i] of `tables` (rows ==
   // nullptr: row i); rows outside [0, n_rows) read row 0.
   const int32_t *rows;
@@ -250,6 +253,11 @@ int attention_part_policy(int elem, int group, int n_kv_heads, bool valu);
 constexpr size_t kPartsBytes = size_t{32} << 20;
 int attention_subs(int elem, int head_dim, int group, int n_kv_heads, bool valu, int64_t n, int max_parts,
                    int max_part, int cu_count);
+// Untuned f16 shapes on the matrix cores (attn_wide_kernel), and the parts per
+// query of a launch (AttnArgs::wide_parts): 0 where the states of n queries'
+// parts exceed kPartsBytes.
+bool attention_wide(int elem, int head_dim, int group, bool valu);
+int attention_wide_parts(int64_t n, int n_heads, int head_dim, int64_t max_len);
 hipError_t launch_decode_attention(const PoolGeom &g, const AttnArgs &a, hipStream_t s);
 
 // One work-group of shared-prefix attention (mq_attn_kernel): the query rows

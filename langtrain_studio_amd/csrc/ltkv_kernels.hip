@@ -24,6 +24,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 #include <type_traits>
@@ -3825,6 +3826,373 @@ attn_any_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const 
 }
 
 // ----------------------------------------------------------------------------
+// Kernel 4 for f16 pools of other shapes (head_dim up to 256 in multiples of
+// 8, any group) on the matrix cores. Bound by memory latency at the sizes
+// such models decode: a work-group is four waves on (query, kv head, up to 16
+// query heads, part of the context), and the parts (wide_part: a
+// function of the query's length) spread one query over the chip. Against attn_any_kernel, which reads a context once per query
+// head and one element per thread: 12 queries of 300-4000 tokens, 32 / 8
+// heads of 96, 1405 us -> 22 us (the launch's bytes: 13 us at 6.5 TB/s).
+//
+// Products as in attn_mfma_kernel, with HDP = head_dim padded to a template
+// width (columns past head_dim load as zeros) and the hi and lo parts of Q
+// and P as operands of their own, so that all 16 columns hold query heads:
+//   S^T[token][head] = K Q^T    A = K rows, loaded straight in the A layout
+//   O^T[d][head]    += V^T P^T  A = V^T through LDS and ds_read_b64_tr_b16
+// The lo products take K and V with non-finite elements clamped: an infinite
+// element times a lo part of the other sign would turn an infinity (or a
+// weight of zero) of the f32 computation into a NaN.
+//
+// A part's state is the left fold of its four waves' states, a query's of its
+// parts' (fold_weights); `max_parts` 0 has the work-group stream and fold the
+// whole context itself, with the same bits (launches whose part states do not
+// fit the buffer).
+// ----------------------------------------------------------------------------
+constexpr int kWideWaves = 4;
+constexpr int kWideParts = 32;
+
+// Tokens per part: 16 parts up to 4096 tokens (of 128 tokens at least), 256
+// tokens up to 8192, 32 parts beyond. Listed launch above, us: 37 with 64
+// tokens at least and 32 parts, 31 so; 256 tokens at least cost one query of
+// 300 tokens, 8 heads of 256, 18 against 15.5 us, 16 parts beyond 4096 one of
+// 8000 tokens 25 against 22.
+__host__ __device__ inline int wide_part(int64_t len) {
+  int64_t p = ((len + 15) / 16 + 63) / 64 * 64;
+  if (p > 256) p = 256;
+  const int64_t most = ((len + kWideParts - 1) / kWideParts + 63) / 64 * 64;
+  if (p < most) p = most;
+  return p < 128 ? 128 : (int)p;
+}
+
+__device__ __forceinline__ h8 finite_h8(const h8 &x) {
+  const h8 top = h8{65504.f16, 65504.f16, 65504.f16, 65504.f16, 65504.f16, 65504.f16, 65504.f16, 65504.f16};
+  return __builtin_elementwise_max(__builtin_elementwise_min(x, top), -top);
+}
+
+__device__ __forceinline__ h4 finite_h4(const h4 &x) {
+  const h4 top = h4{65504.f16, 65504.f16, 65504.f16, 65504.f16};
+  return __builtin_elementwise_max(__builtin_elementwise_min(x, top), -top);
+}
+
+template <int HDP>
+__global__ void __launch_bounds__(64 * kWideWaves)
+attn_wide_kernel(const _Float16 *__restrict__ kpool, const _Float16 *__restrict__ vpool,
+                 const float *__restrict__ q, const int32_t *__restrict__ tables, int64_t table_stride,
+                 const int32_t *__restrict__ lens, float *__restrict__ out, float *__restrict__ part_o,
+                 float *__restrict__ part_ml, int n_kv_heads, int group, int chunks, int head_dim,
+                 int64_t n_blocks, int64_t kv_dim, float qscale, int max_parts,
+                 const int32_t *__restrict__ qmap, const int32_t *__restrict__ rows, int64_t n_rows,
+                 int64_t max_len, int32_t *__restrict__ status) {
+  constexpr int KS = HDP / 32, DT = HDP / 16;
+  constexpr int HP = HDP / 8;              // 16-byte pieces of a padded row
+  constexpr int NLD = (16 * HP + 63) / 64;  // V loads per tile
+  constexpr int VPITCH = HDP * 2 + 32;
+  constexpr int DPW = (DT + kWideWaves - 1) / kWideWaves;  // O tiles a wave folds
+  constexpr uint32_t kOut = 0x7fffffffu;   // an offset outside every extent: reads zero
+  __shared__ __attribute__((aligned(16))) char sv_w[kWideWaves][16 * VPITCH];
+  __shared__ __attribute__((aligned(16))) f32x4 so[kWideWaves][DT][64];
+  __shared__ float sml[kWideWaves][2][16];
+
+  const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int n_heads = n_kv_heads * group;
+  const uint32_t per_query = (uint32_t)n_kv_heads * (uint32_t)chunks;
+  const int hg = (int)(blockIdx.x % per_query);
+  const uint32_t rest = blockIdx.x / per_query;
+  const int part = max_parts > 0 ? (int)(rest % (uint32_t)max_parts) : 0;
+  const int64_t qx = max_parts > 0 ? rest / (uint32_t)max_parts : rest;
+  const int kvh = hg / chunks, head0 = (hg - kvh * chunks) * 16;  // first query head in the group
+  const int64_t qi = qmap ? qmap[qx] : qx;
+  int64_t len = lens[qi];
+  if (len < 0) len = 0;
+  if (len > max_len) len = max_len;
+  const int pt = wide_part(len);
+  const int np = len > 0 ? div_up_tokens(len, pt) : 1;
+  if (part >= np) return;  // uniform
+  const int p_end = max_parts > 0 ? part + 1 : np;
+  const bool live_head = head0 + lr < group;
+  const int64_t qh = qi * n_heads + (int64_t)kvh * group + head0 + (live_head ? lr : 0);
+
+  // B operands: 8 consecutive d of k step ks at d = 32 ks + 8 lq, as hi and
+  // lo parts (heads past the f16 range scaled by 2^-e: q_range_exp).
+  h8 qhi[KS], qlo[KS];
+  float x[KS][8], amax = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int d = 32 * ks + 8 * lq;
+    f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+    if (live_head && d < head_dim) {
+      const float *qp = q + qh * head_dim + d;
+      a = *reinterpret_cast<const f32x4 *>(qp);
+      b = *reinterpret_cast<const f32x4 *>(qp + 4);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      x[ks][e] = (e < 4 ? a[e] : b[e - 4]) * qscale;
+      amax = __builtin_fmaxf(amax, __builtin_fabsf(x[ks][e]));
+    }
+  }
+  const int qex = q_range_exp(rows_reduce<true>(amax));
+  const float qinv = __builtin_ldexpf(1.f, -qex), qmul = __builtin_ldexpf(1.f, qex);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float y = x[ks][e] * qinv;
+      qhi[ks][e] = (_Float16)y;
+      qlo[ks][e] = (_Float16)(y - (float)qhi[ks][e]);
+    }
+
+  const int32_t *tab = table_of(tables, table_stride, rows, n_rows, qi);
+  const uint32_t row_bytes = (uint32_t)(kv_dim * 2);
+  const int64_t block_bytes = 16 * kv_dim * 2;
+  const char *kbase = reinterpret_cast<const char *>(kpool + (int64_t)kvh * head_dim);
+  const char *vbase = reinterpret_cast<const char *>(vpool + (int64_t)kvh * head_dim);
+  uint32_t koff[KS], voff[NLD], vlds[NLD];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int d = 32 * ks + 8 * lq;
+    koff[ks] = d < head_dim ? (uint32_t)lr * row_bytes + (uint32_t)d * 2 : kOut;
+  }
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) {
+    const int idx = i * 64 + lane, r = idx / HP, c = idx - r * HP;
+    voff[i] = r < 16 && c * 8 < head_dim ? (uint32_t)r * row_bytes + (uint32_t)c * 16 : kOut;
+    vlds[i] = (uint32_t)((r < 16 ? r : 15) * VPITCH + (r < 16 ? c * 16 : HDP * 2));  // past the tile: the row's pad
+  }
+  char *sv = sv_w[wave];
+
+  struct Stage {
+    u32x4 k[KS], v[NLD];
+  };
+  // Tile b through descriptors that end at the last row inside the context:
+  // rows past it (and tiles past the part, live false) read as zeros. A table
+  // entry outside the pool reads block 0 (reported by check_table).
+  auto load_tile = [&](int b, int64_t tok1, int b1, Stage &st) __attribute__((always_inline)) {
+    int32_t blk = 0;
+    int ext = 0;
+    if (b < b1) {  // uniform
+      blk = scalar_read(tab, b);
+      if (blk < 0 || blk >= n_blocks) blk = 0;
+      const int valid = (int)(tok1 - (int64_t)b * 16);
+      ext = ((valid < 16 ? valid : 16) - 1) * (int)row_bytes + head_dim * 2;
+    }
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(kbase + (int64_t)blk * block_bytes), (short)0, ext, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(vbase + (int64_t)blk * block_bytes), (short)0, ext, kBufferWord3);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) st.k[ks] = BufVec<16>::template load<0>(rk, koff[ks]);
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) st.v[i] = BufVec<16>::template load<0>(rv, voff[i]);
+  };
+
+  float m_ref, l_run;
+  f32x4 acc[DT];
+  auto compute_tile = [&](int b, int64_t tok1, const Stage &st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) *reinterpret_cast<u32x4 *>(sv + vlds[i]) = st.v[i];
+    f32x4 s = {0.f, 0.f, 0.f, 0.f}, sl = s;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const h8 k = __builtin_bit_cast(h8, st.k[ks]);
+      s = __builtin_amdgcn_mfma_f32_16x16x32_f16(k, qhi[ks], s, 0, 0, 0);
+      sl = __builtin_amdgcn_mfma_f32_16x16x32_f16(finite_h8(k), qlo[ks], sl, 0, 0, 0);
+    }
+    const int valid = (int)(tok1 - (int64_t)b * 16);
+    float sc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sc[i] = (s[i] + sl[i]) * qmul;
+      if (4 * lq + i >= valid) sc[i] = -INFINITY;
+    }
+    const float lmax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(sc[0], sc[1]),
+                                                     __builtin_elementwise_maximum(sc[2], sc[3]));
+    if (__builtin_amdgcn_ballot_w64(lmax > m_ref + kDecodeSlack)) {
+      const float mx = rows_reduce<true>(lmax);
+      if (mx > m_ref + kDecodeSlack) {
+        const float alpha = __builtin_amdgcn_exp2f(m_ref - mx);
+        m_ref = mx;
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
+      }
+    }
+    const float off = m_ref == -INFINITY ? 0.f : m_ref;
+    h4 ph, pl;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p = __builtin_amdgcn_exp2f(sc[i] - off);
+      l_run += p;
+      ph[i] = (_Float16)p;
+      pl[i] = (_Float16)(p - (float)ph[i]);
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const h4 v = __builtin_bit_cast(h4, lds_read_tr(sv + (4 * lq + (lr >> 2)) * VPITCH + (dt * 16 + 4 * (lr & 3)) * 2));
+      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(v, ph, acc[dt], 0, 0, 0);
+      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(finite_h4(v), pl, acc[dt], 0, 0, 0);
+    }
+  };
+
+  // The folded state of the work-group's parts: O tiles wave, wave + 4, ...
+  // (rows d = 16 dt + 4 lq + i, query head head0 + lr).
+  float m_all = -INFINITY, l_all = 0.f;
+  f32x4 o_all[DPW];
+#pragma unroll
+  for (int u = 0; u < DPW; ++u) o_all[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int p = part; p < p_end; ++p) {
+    const int64_t tok0 = (int64_t)p * pt;
+    const int64_t tok1 = len < tok0 + pt ? len : tok0 + pt;
+    const int b0 = (int)(tok0 >> 4), b1 = (int)((tok1 + 15) >> 4);
+    if (wave == 0) check_table(tab, b0, b1, n_blocks, rows, n_rows, qi, status);
+    m_ref = -INFINITY;
+    l_run = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int b = b0 + wave;
+    if (b < b1) {
+      Stage s0, s1;
+      load_tile(b, tok1, b1, s0);
+      for (;;) {
+        load_tile(b + kWideWaves, tok1, b1, s1);
+        compute_tile(b, tok1, s0);
+        if ((b += kWideWaves) >= b1) break;
+        load_tile(b + kWideWaves, tok1, b1, s0);
+        compute_tile(b, tok1, s1);
+        if ((b += kWideWaves) >= b1) break;
+      }
+    }
+    l_run = rows_reduce<false>(l_run);
+    if (p > part) __syncthreads();  // the last part's readers
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) so[wave][dt][lane] = acc[dt];
+    if (lq == 0) {
+      sml[wave][0][lr] = m_ref;
+      sml[wave][1][lr] = l_run;
+    }
+    __syncthreads();
+    // the four waves' states, then the part into the query's
+    float m = -INFINITY, l = 0.f;
+    f32x4 o[DPW];
+#pragma unroll
+    for (int u = 0; u < DPW; ++u) o[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kWideWaves; ++w) {
+      const FoldWeights f = fold_weights(m, sml[w][0][lr]);
+      m = f.m;
+      l = fold_value(f, l, sml[w][1][lr]);
+#pragma unroll
+      for (int u = 0; u < DPW; ++u)
+        if (wave + kWideWaves * u < DT) o[u] = fold_value(f, o[u], so[w][wave + kWideWaves * u][lane]);
+    }
+    if (max_parts > 0) {
+      m_all = m;
+      l_all = l;
+#pragma unroll
+      for (int u = 0; u < DPW; ++u) o_all[u] = o[u];
+    } else {
+      const FoldWeights f = fold_weights(m_all, m);
+      m_all = f.m;
+      l_all = fold_value(f, l_all, l);
+#pragma unroll
+      for (int u = 0; u < DPW; ++u) o_all[u] = fold_value(f, o_all[u], o[u]);
+    }
+  }
+  if (!live_head) return;
+  if (max_parts > 0) {
+    const int64_t pi = qh * max_parts + part;
+#pragma unroll
+    for (int u = 0; u < DPW; ++u) {
+      const int d = 16 * (wave + kWideWaves * u) + 4 * lq;
+      if (d < head_dim) *reinterpret_cast<f32x4 *>(part_o + pi * head_dim + d) = o_all[u];
+    }
+    if (wave == 0 && lq == 0) {
+      part_ml[2 * pi] = m_all;
+      part_ml[2 * pi + 1] = l_all;
+    }
+    return;
+  }
+  const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
+#pragma unroll
+  for (int u = 0; u < DPW; ++u) {
+    const int d = 16 * (wave + kWideWaves * u) + 4 * lq;
+    if (d < head_dim)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[qh * head_dim + d + i] = o_all[u][i] * inv;
+  }
+}
+
+// The left fold of a query's part states: a wave per (query, head), 4 output
+// elements a lane, eight parts' loads in flight.
+__global__ void __launch_bounds__(256)
+attn_wide_merge_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml,
+                       const int32_t *__restrict__ lens, float *__restrict__ out, int n_heads, int head_dim,
+                       int max_parts, int64_t max_len, const int32_t *__restrict__ qmap, int64_t n_pairs) {
+  const int64_t pair = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (pair >= n_pairs) return;
+  const int h = (int)(pair % n_heads);
+  const int64_t qx = pair / n_heads;
+  const int64_t qi = qmap ? qmap[qx] : qx;
+  const int64_t qh = qi * n_heads + h;
+  const int d = (int)(threadIdx.x & 63) * 4;
+  const int dc = d < head_dim ? d : 0;
+  const float *ml = part_ml + 2 * qh * max_parts, *po = part_o + qh * max_parts * head_dim + dc;
+  float mr[8], lr[8];
+  f32x4 orr[8];
+  auto load = [&](int p0) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int p = p0 + u < max_parts ? p0 + u : max_parts - 1;
+      mr[u] = ml[2 * p];
+      lr[u] = ml[2 * p + 1];
+      orr[u] = *reinterpret_cast<const f32x4 *>(po + (int64_t)p * head_dim);
+    }
+  };
+  load(0);  // before the length is known; parts past the query's are not used
+  int64_t len = lens[qi];
+  if (len < 0) len = 0;
+  if (len > max_len) len = max_len;
+  const int np = len > 0 ? div_up_tokens(len, wide_part(len)) : 1;
+  float m = -INFINITY, l = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < np; p0 += 8) {
+    if (p0 > 0) load(p0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (p0 + u < np) {
+        const FoldWeights f = fold_weights(m, mr[u]);
+        m = f.m;
+        l = fold_value(f, l, lr[u]);
+        o = fold_value(f, o, orr[u]);
+      }
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (d < head_dim)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[qh * head_dim + d + i] = o[i] * inv;
+}
+
+template <int HDP>
+hipError_t launch_attn_wide_t(const PoolGeom &g, const AttnArgs &a, hipStream_t s) {
+  const int group = a.n_heads / a.n_kv_heads, chunks = (group + 15) / 16;
+  const int64_t grid = a.n * a.n_kv_heads * chunks * (a.wide_parts > 0 ? a.wide_parts : 1);
+  if (grid >= (int64_t{1} << 32)) return hipErrorInvalidValue;
+  attn_wide_kernel<HDP><<<(unsigned)grid, 64 * kWideWaves, 0, s>>>(
+      static_cast<const _Float16 *>(a.k_layer), static_cast<const _Float16 *>(a.v_layer), a.q, a.tables,
+      a.table_stride, a.lens, a.out, a.part_o, a.part_ml, a.n_kv_heads, group, chunks, a.head_dim, g.n_blocks,
+      g.kv_dim, a.scale * kLog2e, a.wide_parts, a.qmap, a.rows, a.n_rows, a.max_len, a.status);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.wide_parts == 0) return e;
+  const int64_t pairs = a.n * a.n_heads;
+  attn_wide_merge_kernel<<<(unsigned)((pairs + 3) / 4), 256, 0, s>>>(a.part_o, a.part_ml, a.lens, a.out, a.n_heads,
+                                                                     a.head_dim, a.wide_parts, a.max_len, a.qmap,
+                                                                     pairs);
+  return hipGetLastError();
+}
+
+// ----------------------------------------------------------------------------
 // Resident block tables (step descriptor): in-place updates and the slot
 // mapping of a batch's tokens.
 
@@ -4112,6 +4480,17 @@ bool attention_supported(int elem, int head_dim, int group) {
   return (elem == 1 || elem == 2 || elem == 4) && head_dim >= 1 && head_dim <= kAnyMaxHeadDim && group >= 1;
 }
 
+bool attention_wide(int elem, int head_dim, int group, bool valu) {
+  return elem == 2 && !valu && head_dim % 8 == 0 && head_dim <= 256 && !attention_tuned(elem, head_dim, group);
+}
+
+int attention_wide_parts(int64_t n, int n_heads, int head_dim, int64_t max_len) {
+  // most parts of a query of up to max_len tokens (wide_part)
+  const int64_t parts = std::max(std::min<int64_t>((max_len + 127) / 128, 16),
+                                 std::min<int64_t>((max_len + 255) / 256, kWideParts));
+  return n * n_heads * parts * (head_dim + 2) * 4 <= (int64_t)kPartsBytes ? (int)parts : 0;
+}
+
 template <typename T>
 hipError_t launch_attn_any_t(const PoolGeom &g, const AttnArgs &a, hipStream_t s) {
   const int64_t grid = a.n * a.n_heads;
@@ -4135,6 +4514,14 @@ hipError_t launch_decode_attention(const PoolGeom &g, const AttnArgs &a, hipStre
     // the generic kernel takes whole contexts: no partials, no group partials
     if (a.pre_parts || !attention_supported(g.elem, a.head_dim, a.n_heads / a.n_kv_heads))
       return hipErrorInvalidValue;
+    if (attention_wide(g.elem, a.head_dim, a.n_heads / a.n_kv_heads, a.valu)) {
+      if (a.head_dim <= 32) return launch_attn_wide_t<32>(g, a, s);
+      if (a.head_dim <= 64) return launch_attn_wide_t<64>(g, a, s);
+      if (a.head_dim <= 96) return launch_attn_wide_t<96>(g, a, s);
+      if (a.head_dim <= 128) return launch_attn_wide_t<128>(g, a, s);
+      if (a.head_dim <= 192) return launch_attn_wide_t<192>(g, a, s);
+      return launch_attn_wide_t<256>(g, a, s);
+    }
     if (g.elem == 1) return launch_attn_any_t<int8_t>(g, a, s);
     if (g.elem == 2) return launch_attn_any_t<_Float16>(g, a, s);
     return launch_attn_any_t<float>(g, a, s);
