@@ -240,7 +240,7 @@ LTKV_API int ltkv_decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t
  * until the process ends) instead of the cache's workspace, which
  * ltkv_decode_attention grows with hipMalloc on demand. (Launches small
  * enough to run one wave per part of a partition keep their partials in a
- * 32 MiB buffer that every device cache holds from its creation, on either
+ * 64 MiB buffer that every device cache holds from its creation, on either
  * entry point.) A launch whose
  * partials need more fails with LTKV_ERR_ARG before anything is enqueued:
  * they take n * n_heads * P * (head_dim + 2) * 4 bytes, P counted for the

@@ -77,6 +77,8 @@ struct AttnPlan {
   uint64_t groups = 0, grouped = 0, shared_blocks = 0;
   bool groups_only = false;  // every query completed by its group: no per-query pass
   size_t n_pass = 0;         // queries of the per-query pass (the rest are completed by groups)
+  size_t n_plain = 0;        // ... of which the first n_plain of the query map have no group partials
+  bool separate = false;     // ... and the others nothing but group partials: two launches
   size_t max_suffix = 0;     // longest remainder (tokens) of a per-query-pass query
   bool empty_with_groups = false;  // a query with group partials and no remainder
   bool pass_empty = false;         // every per-query-pass query is such a query
@@ -143,8 +145,8 @@ struct ltkv_cache {
   // Attention workspace (partition partials), grown on demand.
   uint8_t *ws = nullptr;
   size_t ws_bytes = 0;
-  // Partials of small launches (ltkv::kPartsBytes, held from creation): the
-  // states of parts, and partition partials of up to half its size.
+  // Partials of small launches, held from creation: ltkv::kPartsBytes for the
+  // states of parts, as many for partition and group partials.
   uint8_t *parts = nullptr;
   // The device's static scratch (ltkv_decode_attention_noalloc), looked up at
   // creation; shared by every cache on the device.
@@ -422,12 +424,13 @@ int ensure_workspace(ltkv_cache *c, size_t bytes) {
   return LTKV_OK;
 }
 
-// Memory for a launch's partials: the buffer held from the cache's creation
-// for up to half of it (no allocation on a first call; the launches of a
-// cache follow each other on its stream), the workspace beyond.
-int workspace(ltkv_cache *c, size_t bytes, uint8_t **base) {
-  if (bytes <= ltkv::kPartsBytes / 2) {
-    *base = c->parts;
+// Memory for a launch's partials: up to `limit` bytes (at most kPartsBytes) of
+// the buffer held from the cache's creation, after the parts' states (no
+// allocation on a first call; the launches of a cache follow each other on
+// its stream), the workspace beyond.
+int workspace(ltkv_cache *c, size_t bytes, size_t limit, uint8_t **base) {
+  if (bytes <= limit) {
+    *base = c->parts + ltkv::kPartsBytes;
     return LTKV_OK;
   }
   if (int rc = ensure_workspace(c, bytes)) return rc;
@@ -874,10 +877,18 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
     return fail(LTKV_ERR_ARG, "block tables of this batch are too large");
   std::vector<int32_t> qmap;  // queries left for the per-query pass
   size_t max_suffix = 0;
-  bool empty_with_groups = false, pass_empty = true;
+  bool empty_with_groups = false, pass_empty = true, separate = true;
+  // Queries without group partials first, then those with some.
+  for (size_t i = 0; i < n; ++i)
+    if (pre_parts[i] == 0) qmap.push_back((int32_t)i);
+  const size_t n_plain = qmap.size();
+  for (size_t i = 0; i < n; ++i)
+    if (pre_parts[i] > 0) {
+      qmap.push_back((int32_t)i);
+      if (lens[i] > pre_tokens[i]) separate = false;
+    }
   for (size_t i = 0; i < n; ++i)
     if (pre_parts[i] >= 0) {
-      qmap.push_back((int32_t)i);
       const size_t rem = lens[i] > pre_tokens[i] ? lens[i] - pre_tokens[i] : 0;
       max_suffix = std::max(max_suffix, rem);
       if (pre_parts[i] > 0 && rem == 0) empty_with_groups = true;
@@ -897,6 +908,8 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
   P.shared_blocks = shared_blocks;
   P.groups_only = groups_only;
   P.n_pass = qmap.size();
+  P.n_plain = n_plain;
+  P.separate = separate && n_plain > 0;
   P.max_suffix = max_suffix;
   P.empty_with_groups = empty_with_groups;
   P.pass_empty = pass_empty && !groups_only;
@@ -1045,7 +1058,7 @@ int ltkv_create(size_t n_layers, size_t kv_dim, size_t n_tokens, int dtype, int 
     if ((e = hipMalloc((void **)&c->d_status, 4 * sizeof(int32_t))) != hipSuccess) rc = hip_fail(e, "hipMalloc(status)");
     else if ((e = hipMemset(c->d_status, 0, 4 * sizeof(int32_t))) != hipSuccess) rc = hip_fail(e, "hipMemset(status)");
   }
-  if (rc == LTKV_OK && (e = hipMalloc((void **)&c->parts, ltkv::kPartsBytes)) != hipSuccess)
+  if (rc == LTKV_OK && (e = hipMalloc((void **)&c->parts, 2 * ltkv::kPartsBytes)) != hipSuccess)
     rc = hip_fail(e, "hipMalloc(parts)");
   const size_t sbytes = c->q8() ? n_layers * c->layer_scales() * 2 : 0;
   if (rc == LTKV_OK && sbytes > 0) {
@@ -1508,7 +1521,7 @@ int decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, size
                   (long long)ws.bytes, ltkv::kScratchBytes);
     base = c->scratch;
   } else if (subs == 0) {
-    if (int rc = workspace(c, (size_t)ws.bytes, &base)) return rc;
+    if (int rc = workspace(c, (size_t)ws.bytes, ltkv::kPartsBytes / 2, &base)) return rc;
   }
   if (subs > 0) {
     ws = ltkv::attention_workspace((int64_t)n, (int)n_heads, (int)head_dim, (int)max_parts * subs, true);
@@ -1752,30 +1765,21 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
 
   DeviceGuard dg(c->device);
   if (!dg.ok) return fail(LTKV_ERR_HIP, "hipSetDevice(%d) failed", c->device);
+  // (no partition partials where the groups cover every query's context)
   ltkv::AttnWorkspace ws = ltkv::attention_workspace(
-      (int64_t)P.n, (int)P.n_heads, (int)P.head_dim, (int)max_parts, grouped);
+      (int64_t)P.n, (int)P.n_heads, (int)P.head_dim, (int)max_parts, grouped && !P.pass_empty && !P.groups_only);
+  if (grouped && (P.pass_empty || P.groups_only)) ws = ltkv::AttnWorkspace{0, 0, 0};
   const size_t pre_slots = grouped ? P.n * P.n_heads * (size_t)P.max_pre_parts : 0;
   const size_t pre_o_off = ((size_t)ws.bytes + 255) / 256 * 256;
   const size_t pre_ml_off = pre_o_off + pre_slots * P.head_dim * 4;
   uint8_t *base = nullptr;
-  if (int rc = workspace(c, pre_ml_off + pre_slots * 2 * 4, &base)) return rc;
+  if (int rc = workspace(c, pre_ml_off + pre_slots * 2 * 4, ltkv::kPartsBytes, &base)) return rc;
   const int32_t *d = reinterpret_cast<const int32_t *>(P.d);
   const ltkv::PoolGeom g = head_geom(c, P.head_dim);
   ltkv::AttnArgs a = attn_args(c, layer, P.n, P.n_heads, P.head_dim, scale, d_q, d_out, ws, part,
                                (int)max_parts, base);
   a.split = split;
   set_wide_parts(c, a, group, P.sstride * LTKV_BLOCK);
-  if (!grouped) {  // a plain decode batch: its small launches as decode_attention's
-    a.subs = ltkv::attention_subs((int)c->elem, (int)P.head_dim, (int)group, a.n_kv_heads, a.valu, a.n,
-                                  (int)max_parts,
-                                  ltkv::max_partition_size((int64_t)(P.sstride * LTKV_BLOCK), part, split),
-                                  c->device_count_cu);
-    if (a.subs > 0) {
-      ws = ltkv::attention_workspace(a.n, a.n_heads, a.head_dim, (int)max_parts * a.subs, true);
-      a.part_o = (float *)(c->parts + ws.part_o_off);
-      a.part_ml = (float *)(c->parts + ws.part_ml_off);
-    }
-  }
   // Short remainders in one partition each and no group-only queries: the
   // decode kernel writes every output itself (folding group partials).
   a.merge_free = grouped && part > 0 && P.max_suffix <= (size_t)(part / split) && !P.empty_with_groups;
@@ -1816,6 +1820,39 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
     // footprint (two waves per SIMD) leaves no room to overlap them.
     HIP_TRY(ltkv::launch_mq_attention(g, m, c->stream), "shared-prefix attention launch");
     if (P.groups_only) return LTKV_OK;  // the groups wrote every output
+  }
+  // Small launches as decode_attention's.
+  auto set_subs = [&](ltkv::AttnArgs &w) {
+    w.subs = ltkv::attention_subs((int)c->elem, (int)P.head_dim, (int)group, w.n_kv_heads, w.valu, w.n,
+                                  (int)max_parts,
+                                  ltkv::max_partition_size((int64_t)(P.sstride * LTKV_BLOCK), part, split),
+                                  c->device_count_cu);
+    if (w.subs > 0) {
+      const ltkv::AttnWorkspace pw =
+          ltkv::attention_workspace(w.n, w.n_heads, w.head_dim, (int)max_parts * w.subs, true);
+      w.part_o = (float *)(c->parts + pw.part_o_off);
+      w.part_ml = (float *)(c->parts + pw.part_ml_off);
+    }
+  };
+  if (!grouped) {
+    set_subs(a);
+  } else if (P.separate && !a.valu) {
+    // Decodes beside prompt chunks that are cut into ranges: the decodes as a
+    // plain batch, then the chunks' merge. In one pass, every chunk query
+    // started waves of the decode kernel that found nothing to read, and the
+    // batch was too large for the longest-first order.
+    ltkv::AttnArgs w = a;
+    w.n = (int64_t)P.n_plain;
+    w.qmap = d + P.off_qmap;
+    w.pre_parts = nullptr;
+    w.merge_free = false;
+    set_subs(w);
+    HIP_TRY(ltkv::launch_decode_attention(g, w, c->stream), "decode attention launch");
+    if (P.n_pass == P.n_plain) return LTKV_OK;
+    a.n = (int64_t)(P.n_pass - P.n_plain);
+    a.qmap = d + P.off_qmap + P.n_plain;
+    a.merge_free = false;
+    a.pass_empty = true;
   }
   HIP_TRY(ltkv::launch_decode_attention(g, a, c->stream), "decode attention launch");
   return LTKV_OK;

@@ -984,7 +984,9 @@ __device__ __forceinline__ void merge_add(float a, float l, const f32x4 &po, flo
 // threads with 4 output elements each (16-byte loads and stores), a
 // work-group 256 / (HD/4) pairs; the partition loop is unrolled so several
 // partials are in flight per thread.
-template <int HD, int NF>
+// GROUPS: only group partials (AttnArgs::pass_empty); the first NF of them
+// are loaded up front instead.
+template <int HD, int NF, bool GROUPS>
 __global__ void __launch_bounds__(256)
 attn_merge_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml,
                   const int32_t *__restrict__ lens, float *__restrict__ out, int n_heads,
@@ -1010,12 +1012,14 @@ attn_merge_kernel(const float *__restrict__ part_o, const float *__restrict__ pa
   f32x4 o4[NF];
 #pragma unroll
   for (int p = 0; p < NF; ++p) {
-    const int pc = p < max_parts ? p : max_parts - 1;
-    m4[p] = ml[2 * pc];
-    l4[p] = ml[2 * pc + 1];
-    o4[p] = *reinterpret_cast<const f32x4 *>(part_o + (qh * max_parts + pc) * HD + d);
+    const int most = GROUPS ? max_pre_parts : max_parts;
+    const int pc = p < most ? p : most - 1;
+    const float *pm = GROUPS ? pre_ml + qh * most * 2 : ml;
+    m4[p] = pm[2 * pc];
+    l4[p] = pm[2 * pc + 1];
+    o4[p] = *reinterpret_cast<const f32x4 *>((GROUPS ? pre_o : part_o) + (qh * most + pc) * HD + d);
   }
-  int64_t len = lens[qi];
+  int64_t len = GROUPS ? 0 : lens[qi];
   if (len < 0) len = 0;
   if (len > max_len) len = max_len;
   const int pt = split_partition(len, part_tokens, split);
@@ -1027,17 +1031,18 @@ attn_merge_kernel(const float *__restrict__ part_o, const float *__restrict__ pa
   const int np = div_up_tokens(len, pt);
   if (np <= 1 && npre == 0) return;
   if (np == 1 && folded) return;
-  if (npre == 0 && np <= NF) {
-    // The common case (a query of up to NF partitions, np <= max_parts).
+  const int nf = GROUPS ? npre : np;
+  if ((GROUPS || npre == 0) && nf <= NF) {
+    // The common case (a query of up to NF partials, all loaded).
     float mx = m4[0];
 #pragma unroll
-    for (int p = 1; p < NF; ++p) mx = p < np ? __builtin_fmaxf(mx, m4[p]) : mx;
+    for (int p = 1; p < NF; ++p) mx = p < nf ? __builtin_fmaxf(mx, m4[p]) : mx;
     const float mref = mx == -INFINITY ? 0.f : mx;
     float lsum = 0.f;
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int p = 0; p < NF; ++p) {
-      if (p < np) {
+      if (p < nf) {
         const float a = __builtin_amdgcn_exp2f(m4[p] - mref);
         merge_add(a, l4[p], o4[p], lsum, o);
       }
@@ -1079,7 +1084,8 @@ hipError_t launch_merge(const AttnArgs &a, hipStream_t s, bool folded) {
   constexpr int ppw = 256 / (HD / 4);
   const unsigned mgrid = (unsigned)((pairs + ppw - 1) / ppw);
   // One round of loads for queries of up to four (eight) partitions.
-  auto kern = a.max_parts <= 4 ? attn_merge_kernel<HD, 4> : attn_merge_kernel<HD, 8>;
+  auto kern = a.pass_empty ? (a.max_pre_parts <= 4 ? attn_merge_kernel<HD, 4, true> : attn_merge_kernel<HD, 8, true>)
+                           : (a.max_parts <= 4 ? attn_merge_kernel<HD, 4, false> : attn_merge_kernel<HD, 8, false>);
   kern<<<mgrid, 256, 0, s>>>(a.part_o, a.part_ml, a.lens, a.out, a.n_heads, a.part_tokens, a.split, a.max_parts,
                              a.max_len, a.pre_parts, a.pre_o, a.pre_ml, a.max_pre_parts, a.qmap, pairs,
                              folded ? 1 : 0);
@@ -1701,7 +1707,7 @@ attn_merge_subs_kernel(const float *__restrict__ part_o, const float *__restrict
   const int64_t qi = qmap ? qmap[qx] : qx;
   const int64_t qh = qi * n_heads + h;
   const int g = (int)threadIdx.x / TPP, c = (int)threadIdx.x % TPP;
-  const int64_t slot0 = qh * max_parts * subs;
+  const int64_t slot0 = pair * max_parts * subs;
   const float *ml = part_ml + 2 * slot0;
   const float *po = part_o + slot0 * HD + 4 * c;
   float mr[kMergeSubs], lr[kMergeSubs];
@@ -1885,7 +1891,7 @@ struct OrderShapes {
 };
 
 template <bool FIRST_WAVE_COUNTS = false, bool RUNS = false>
-__device__ __forceinline__ int decode_order_setup(const int32_t *__restrict__ lens, int64_t n, int64_t max_len,
+__device__ __forceinline__ int decode_order_setup(const int32_t *__restrict__ lens, const int32_t *__restrict__ qmap, int64_t n, int64_t max_len,
                                                   int part_tokens, int split, int lane, int32_t *hist,
                                                   OrderShapes &sh, int n_groups, int slots, int max_run) {
   if (lane < kOrderClasses) hist[lane] = 0;
@@ -1900,8 +1906,8 @@ __device__ __forceinline__ int decode_order_setup(const int32_t *__restrict__ le
     sh.len[c] = 0;
     pt[c] = 1;
     if ((int64_t)c * 64 + lane < n)
-      decode_query_parts(lens, (int64_t)c * 64 + lane, max_len, part_tokens, split, sh.len[c], pt[c],
-                         sh.items[c]);
+      decode_query_parts(lens, qmap ? qmap[c * 64 + lane] : (int64_t)c * 64 + lane, max_len, part_tokens, split,
+                         sh.len[c], pt[c], sh.items[c]);
   }
   if constexpr (RUNS) {
     // The run length: the shortest whose items all start at once (they then
@@ -2177,7 +2183,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   int run = 1;
   int sub = 0;  // FINE: the wave's part of its partition
   if (!FINE && order)
-    run = decode_order_setup<(NW > 1), RUNS>(lens, n_queries, max_len, part_tokens, split, lane, shist, osh,
+    run = decode_order_setup<(NW > 1), RUNS>(lens, qmap, n_queries, max_len, part_tokens, split, lane, shist, osh,
                                              n_groups, slots, kRunSlots + 1);
 
   // B operands Q'_a^T of the score product, one per kv head a of the wave:
@@ -2286,7 +2292,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   // One item: a partition [tok0, tok1) of query qi (tiles b0 .. b1 - 1).
   // Every field is uniform over the wave (scalar registers).
   struct Item {
-    int64_t qi, len, tok1;
+    int64_t qx, qi, len, tok1;  // qx: the launch's query, qi: the batch's
     int part, np, b0, b1;  // part: the partition of tile b (the item's first one at the start)
     int p0, plast, pt_tiles;  // the item's first and last partitions; tiles per partition
     const int32_t *tab;
@@ -2315,7 +2321,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
     const int64_t qi = qmap ? qmap[qx] : qx;
     int64_t len;
     if (!FINE && order) {
-      len = olen;  // the order scan read and clamped it (ordered launches have no query map)
+      len = olen;  // the order scan read and clamped it
     } else {
       len = lens[qi];
       if (len < 0) len = 0;
@@ -2348,6 +2354,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
       if (sub > 0 && (tok0 >= tend || tok0 >= len)) return;
       tend = tend < tok0 + st ? tend : tok0 + st;
     }
+    it.qx = qx;
     it.qi = qi;
     it.len = len;
     it.part = part;
@@ -2663,7 +2670,8 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   // wave's part of it.
   auto write_partial = [&](const Item &it) __attribute__((always_inline)) {
     if (!hi_lane) return;
-    const int64_t qh = it.qi * n_heads + (int64_t)kvh0 * G + lr;
+    // (FINE: slots by the launch's query, so a query map's launch stays small)
+    const int64_t qh = (FINE ? it.qx : it.qi) * n_heads + (int64_t)kvh0 * G + lr;
     const int64_t pi = FINE ? (qh * max_parts + it.part) * subs + sub : qh * max_parts + it.part;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -2899,11 +2907,13 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   if (fault_q >= 0) report_fault(status, kFaultTable, fault_q);
 }
 
-// Plain decode attention of up to kOrderMaxQueries queries takes its items
-// longest first; planned launches (query maps, group partials) keep query
-// order.
+// Launches of up to kOrderMaxQueries queries take their items longest first;
+// short remainders after group partials (merge_free: one partition each) keep
+// query order, where the scan would cost more than it gives. The 120 decodes
+// of 512-8191 tokens beside eight 512-token chunks (Qwen2.5-7B, one query map
+// entry each): 233 us in query order, 162 us so.
 inline bool decode_ordered(const AttnArgs &a) {
-  return !a.qmap && !a.pre_parts && a.n > 1 && a.n <= kOrderMaxQueries;
+  return !a.merge_free && a.n > 1 && a.n <= kOrderMaxQueries;
 }
 
 // One wave per item (a partition of NH kv heads of one query), kDecodeWaves
