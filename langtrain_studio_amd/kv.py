@@ -50,19 +50,26 @@ def _np_ptr(a: np.ndarray):
     return a.ctypes.data_as(C.c_void_p)
 
 
-def _dev_ptr(t, dtype, name: str, device: int):
-    """Device address of a contiguous torch tensor of the given dtype."""
-    import torch
+_torch = None
 
-    if not isinstance(t, torch.Tensor) or not t.is_cuda:
+
+def _dev_ptr(t, dtype, name: str, device: int) -> int:
+    """Device address of a contiguous torch tensor of the given dtype. A
+    decode call checks seven tensors, ~0.7 us each with the module lookup,
+    ``t.device`` object and ctypes pointer of each, so the good case takes the
+    cheapest form of the same tests."""
+    global _torch
+    if _torch is None:
+        import torch as _torch
+    if not isinstance(t, _torch.Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a HIP device tensor")
-    if t.dtype != dtype:
+    if t.dtype is not dtype:
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    if t.device.index != device:
+    if t.get_device() != device:
         raise ValueError(f"{name} is on {t.device}, cache is on device {device}")
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 class KvCache:
@@ -90,7 +97,9 @@ class KvCache:
         self.elem = {"f16": 2, "f32": 4, "q8_0": 1}[dtype]
         self.device = device
         self.n_blocks = self._lib.ltkv_n_blocks(h)
+        self._kv_dim = self._lib.ltkv_kv_dim(h)
         self._plan_shape = None
+        self._stream = 0
         if stream is not None:
             self.set_stream(stream)
 
@@ -114,13 +123,14 @@ class KvCache:
 
     def set_stream(self, stream) -> None:
         """Enqueue device work on ``stream`` (a torch.cuda.Stream or a raw hipStream_t)."""
-        raw = getattr(stream, "cuda_stream", stream)
-        _check(self._lib.ltkv_set_stream(self._h, C.c_void_p(int(raw or 0))))
+        raw = int(getattr(stream, "cuda_stream", stream) or 0)
+        _check(self._lib.ltkv_set_stream(self._h, C.c_void_p(raw)))
+        self._stream = raw
 
     # ---- kv.rs:17-18,50-60,185-187 --------------------------------------------------
     @property
     def kv_dim(self) -> int:
-        return self._lib.ltkv_kv_dim(self._h)
+        return self._kv_dim
 
     def capacity(self) -> int:
         return self._lib.ltkv_capacity(self._h)
