@@ -591,8 +591,15 @@ void set_wide_parts(const ltkv_cache *c, ltkv::AttnArgs &a, size_t group, size_t
 // Fewest shared full blocks and members for a prefix group.
 constexpr size_t kMinSharedBlocks = 2;
 // Tokens per group partition are at least this (a multiple of the kernel's
-// 32-token staging step).
+// 32-token staging step); prefix groups, whose partials are folded anyway
+// (the chunks of a prompt in one partition write their outputs themselves),
+// take shorter ones up to kShortPrefixParts of them: 31 forks of a 740-token
+// prefix (Qwen2.5-7B, q8_0) 56 us with partitions of 256 tokens, 36 so; 50 of
+// 500 tokens (Llama-3-8B, f16) 43 / 31; prompt chunks of 208 tokens 41 us in
+// one partition, 53 cut into such ones.
 constexpr size_t kMinPrefixPart = 256;
+constexpr size_t kShortPrefixPart = 64;
+constexpr size_t kShortPrefixParts = 8;
 // Longest per-query remainder for which grouped plans size the per-query pass's items themselves.
 constexpr size_t kShortRemainder = 512;
 
@@ -672,6 +679,7 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
     std::vector<int32_t> members;
     size_t tokens;
     int32_t table_query;  // a member whose table covers the range
+    bool causal = false;  // queries of one sequence
   };
   std::vector<Group> groups;
   std::vector<size_t> pre_tokens(n, 0);  // context of query i covered by its group
@@ -719,6 +727,7 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
       for (auto &b : by_seq) {
         if (b.size() < 2) continue;
         Group gr;
+        gr.causal = true;
         gr.table_query = b[0];
         for (int32_t m : b)
           if (lens[m] > lens[gr.table_query]) gr.table_query = m;
@@ -796,7 +805,9 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
   // chunk's jobs alone set the kernel's end, 19% past the mean load).
   size_t work = 0;  // token-rows of all jobs, counted as full ranges
   for (const auto &gr : groups) work += (gr.members.size() + per_job - 1) / per_job * n_kv_heads * gr.tokens;
-  const size_t mean_tokens = std::max<size_t>(1, work / std::max<size_t>(1, target));
+  // (rounded up: a 487-token chunk after 900 tokens was 290 jobs on 256
+  // work-group slots with the mean rounded down, 65 us; 240 jobs, 50 us so)
+  const size_t mean_tokens = std::max<size_t>(1, (work + target - 1) / std::max<size_t>(1, target));
   std::vector<ltkv::MqJob> jobs;
   std::vector<int32_t> members;
   std::vector<int32_t> pre_parts(n, 0);
@@ -807,7 +818,8 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
   for (size_t gi = 0; gi < groups.size(); ++gi) {
     const Group &gr = groups[gi];
     const size_t tokens = gr.tokens;
-    const size_t max_split = std::max<size_t>(1, tokens / kMinPrefixPart);
+    size_t max_split = std::max<size_t>(1, tokens / kMinPrefixPart);
+    if (!gr.causal) max_split = std::max(max_split, std::min(tokens / kShortPrefixPart, kShortPrefixParts));
     const size_t fill = std::max<size_t>((target + units - 1) / units, (tokens + mean_tokens - 1) / mean_tokens);
     const size_t split = std::max(std::min(max_split, std::max<size_t>(1, fill)),
                                   (tokens + ltkv::kMqMaxRange - 1) / ltkv::kMqMaxRange);
