@@ -4583,18 +4583,20 @@ int attention_subs(int elem, int head_dim, int group, int n_kv_heads, bool valu,
   const bool pairs = group <= 4 && n_kv_heads % 2 == 0;  // two kv heads a wave
   const int64_t waves = n * (n_kv_heads / (pairs ? 2 : 1)) * max_parts;
   const int64_t subs = div_up_tokens(max_part, sub_tokens(0, head_dim));
-  // Where the partitions number at most half the SIMDs. Measured (us,
-  // partitions against parts; Llama-3-8B f16): 16 queries of 200-3000 tokens
-  // 80.5 / 32.2, 32 of 2048-4096 (512 partitions) 92-103 / 82; 64 of them
-  // (1024) 129 / 161. head_dim 64 partitions take half the time (TinyLlama,
-  // 256: 36 / 25; 512: 41 / 46), q8_0 waves of one head nearly as long as
-  // f16 ones at half the bytes (Qwen2.5-7B, 512: 69 / 42; 1024: 72 / 69).
-  // Partitions of up to three parts gain only from the work-groups of one
-  // wave, up to one a CU (Qwen2.5-7B q8_0, 1024 of 192 tokens: 26.3 / 27.7).
-  int64_t limit = 2 * (int64_t)cu_count;
-  if (subs < 4) limit = cu_count;
-  else if (head_dim == 64) limit = 3 * (int64_t)cu_count / 2;
+  // Where the partitions number about half the SIMDs or less. Measured (us,
+  // partitions against parts; the lines lie between the last gain and the
+  // first loss): Llama-3-8B f16, 16 queries of 200-3000 tokens 80.5 / 32.2,
+  // 512 partitions 92-103 / 82, 616 of ragged lengths 90 / 64, 768 104 / 121;
+  // q8_0, 768 54 / 47, 1024 56 / 58. head_dim 64: SmolLM2 f16, 768 42 / 34;
+  // TinyLlama f16, 768 38 / 35, 1024 41 / 45. q8_0 waves of one head last
+  // nearly as long as f16 ones at half the bytes (Qwen2.5-7B, 1024 72 / 69;
+  // TinyLlama, 1024 53 / 42). Partitions of up to three parts gain only from
+  // the work-groups of one wave (Llama-3-8B f16, 480 19.0 / 16.4, 896 15 / 20;
+  // Qwen2.5-7B q8_0, 1024 26 / 28).
+  int64_t limit = 5 * (int64_t)cu_count / 2;
+  if (subs < 4) limit = 2 * (int64_t)cu_count;
   else if (elem == 1 && !pairs) limit = 4 * (int64_t)cu_count;
+  else if (elem == 1 || head_dim == 64) limit = 3 * (int64_t)cu_count;
   if (waves > limit) return 0;
   const int64_t bytes = n * n_kv_heads * group * max_parts * subs * (head_dim + 2) * 4;
   return bytes > (int64_t)kPartsBytes ? 0 : (int)subs;
