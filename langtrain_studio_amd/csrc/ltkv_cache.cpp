@@ -1618,10 +1618,9 @@ int ltkv_append_decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t n
   if (src_stride < c->kv_dim || src_stride % 4 != 0)
     return fail(LTKV_ERR_ARG, "src_stride must be >= kv_dim and a multiple of 4");
   if (((uintptr_t)d_k | (uintptr_t)d_v) % 16 != 0) return fail(LTKV_ERR_ARG, "K/V rows must be 16-byte aligned");
-  if (c->elem != 2 || !ltkv::attention_tuned(2, (int)head_dim, (int)group) ||
-      c->attn_engine == LTKV_ENGINE_VALU) {
-    // fused only on f16 pools of the tuned shapes with the matrix-core kernel:
-    // otherwise append, then attention, as two launches
+  if (!ltkv::attention_tuned((int)c->elem, (int)head_dim, (int)group) || c->attn_engine == LTKV_ENGINE_VALU) {
+    // fused on the tuned shapes, except by the vector-ALU kernels on f16
+    // pools: otherwise append, then attention, as two launches
     if (int rc = ltkv_write(c, layer, n, d_slot_mapping, d_k, d_v, src_stride)) return rc;
     return ltkv_decode_attention(c, layer, n, n_heads, head_dim, scale, d_q, d_tables, table_stride,
                                  d_lens, d_out);
