@@ -138,10 +138,10 @@ struct AttnArgs {
   // group partials and an empty remainder, so only the merge runs (it folds
   // the group partials by itself).
   bool pass_empty;
-  // Fused append (f16 pools, matrix-core kernel): query i's new K/V row
-  // (new_k/new_v row i, f32, row stride new_stride) is written to cell
-  // new_slots[i], which must be position lens[i] - 1 of the query's table,
-  // and attended from registers. nullptr: no fused append.
+  // Fused append (tuned kernels; not the vector-ALU ones on f16 pools): query
+  // i's new K/V row (new_k/new_v row i, f32, row stride new_stride) is written
+  // to cell new_slots[i], which must be position lens[i] - 1 of the query's
+  // table, and attended (f16: from registers). nullptr: no fused append.
   const int32_t *new_slots;
   const float *new_k, *new_v;
   int64_t new_stride;
@@ -233,8 +233,9 @@ struct AttnWorkspace {
 AttnWorkspace attention_workspace(int64_t n, int n_heads, int head_dim, int max_parts,
                                   bool always = false);
 // Shapes of the tuned decode kernels (head_dim 64 or 128, group 1..8) and of
-// every kernel (any group, head_dim up to 1024: the generic kernel, one
-// work-group per query head, no partitions, no group partials).
+// every kernel (any group, head_dim up to 1024: attention_wide's shapes, or
+// the generic kernel, one work-group per query head; no partitions, no group
+// partials).
 bool attention_tuned(int elem, int head_dim, int group);
 bool attention_supported(int elem, int head_dim, int group);
 // Decode kernels on f16 and q8_0 pools read two adjacent kv heads per wave

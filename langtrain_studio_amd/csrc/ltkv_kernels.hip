@@ -10,6 +10,10 @@
 //                                       (f16 and q8_0 pools), split over context partitions
 //   attn16_kernel / attn_kernel         the same on the vector ALU (f32 pools)
 //   attn_merge_kernel                   log-sum-exp merge of the partitions (model.rs:431-475)
+//   attn_merge_subs_kernel              the same after a launch of one wave per part
+//   attn_wide_kernel                    decode attention of other f16 shapes on the matrix
+//                                       cores, merged by attn_wide_merge_kernel
+//   attn_any_kernel                     decode attention of any other shape
 //   mq_attn_kernel                      query rows that share K/V rows (prefix groups,
 //                                       prefill chunks) on the matrix cores
 //   table_update_kernel / slot_mapping_kernel  resident block tables and the slot
@@ -1871,9 +1875,9 @@ __device__ __forceinline__ int q_range_exp(float amax) {
 // or uploaded per step on the host; a query's partitions and result bits do
 // not depend on where its items land.
 //
-// When the batch holds at least twice as many partitions (times the kv-head
-// groups) as the chip holds waves at once, an item is a run of k consecutive
-// partitions of one query, k = partitions / wave slots: one wave streams
+// When the batch may hold at least twice as many partitions (times the
+// kv-head groups) as the chip holds waves at once, an item is a run of k <= 4
+// consecutive partitions of one query (decode_order_setup's rule): one wave streams
 // them back to back and writes each partition's partial as it passes its
 // end, so every partial (and every output bit) is the one a wave per
 // partition writes, while each wave pays its start (order scan, first table
@@ -3728,10 +3732,11 @@ mq_attn_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool,
 // takes any shape (model.rs:401-402 reads head_dim and the group from the
 // model; its own cache test uses kv_dim 4, kv.rs:202-229): rows whose byte
 // length is not a multiple of 16 move element by element, and attention with
-// a head_dim other than 64 / 128 or a group above 8 runs on the vector ALU
-// with one work-group per (query, query head). They are correct for any
-// shape and serve the families the tuned kernels do not; the tuned kernels
-// stay the path for every shape they cover.
+// a head_dim other than 64 / 128 or a group above 8 runs on attn_wide_kernel
+// (f16 pools, head_dim up to 256 in multiples of 8) or, on the vector ALU
+// with one work-group per (query, query head), on attn_any_kernel. They are
+// correct for any shape and serve the families the tuned kernels do not; the
+// tuned kernels stay the path for every shape they cover.
 // ----------------------------------------------------------------------------
 
 // Append of one element of K and of V per thread (any kv_dim).

@@ -406,7 +406,7 @@ class KvCache:
     def append_decode_attention(self, layer: int, slot_mapping, k, v, q, tables, lens, n_heads: int,
                                 head_dim: int, scale: Optional[float] = None, out=None):
         """write_batch(layer, slot_mapping, k, v) then decode_attention in one
-        launch (f16 pools): slot_mapping[i] must be position lens[i] - 1 of
+        launch (tuned shapes): slot_mapping[i] must be position lens[i] - 1 of
         query i's table, one new token per sequence."""
         import torch
 
