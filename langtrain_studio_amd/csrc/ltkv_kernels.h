@@ -236,7 +236,10 @@ AttnWorkspace attention_workspace(int64_t n, int n_heads, int head_dim, int max_
 // every kernel (any group, head_dim up to 1024: attention_wide's shapes, or
 // the generic kernel, one work-group per query head; no partitions, no group
 // partials).
-bool attention_tuned(int elem, int head_dim, int group);
+inline bool attention_tuned(int elem, int head_dim, int group) {
+  return (elem == 1 || elem == 2 || elem == 4) && (head_dim == 64 || head_dim == 128) && group >= 1 &&
+         group <= 8;
+}
 bool attention_supported(int elem, int head_dim, int group);
 // Decode kernels on f16 and q8_0 pools read two adjacent kv heads per wave
 // when the group has at most 4 query heads and the kv heads pair up (the
@@ -252,8 +255,66 @@ int attention_part_policy(int elem, int group, int n_kv_heads, bool valu);
 // partition. Their states fit kPartsBytes (of a buffer each cache holds from
 // its creation, so no launch allocates for them).
 constexpr size_t kPartsBytes = size_t{32} << 20;
-int attention_subs(int elem, int head_dim, int group, int n_kv_heads, bool valu, int64_t n, int max_parts,
-                   int max_part, int cu_count);
+inline int attention_subs(int elem, int head_dim, int group, int n_kv_heads, bool valu, int64_t n, int max_parts,
+                          int max_part, int cu_count) {
+  if (elem == 4 || valu || !attention_tuned(elem, head_dim, group)) return 0;
+  const bool pairs = group <= 4 && n_kv_heads % 2 == 0;  // two kv heads a wave
+  const int64_t waves = n * (n_kv_heads / (pairs ? 2 : 1)) * max_parts;
+  const int64_t subs = div_up_tokens(max_part, sub_tokens(0, head_dim));
+  // Where the partitions number about half the SIMDs or less. Measured (us,
+  // partitions against parts; the lines lie between the last gain and the
+  // first loss): Llama-3-8B f16, 16 queries of 200-3000 tokens 80.5 / 32.2,
+  // 512 partitions 92-103 / 82, 616 of ragged lengths 90 / 64, 768 104 / 121;
+  // q8_0, 768 54 / 47, 1024 56 / 58. head_dim 64: SmolLM2 f16, 768 42 / 34;
+  // TinyLlama f16, 768 38 / 35, 1024 41 / 45. q8_0 waves of one head last
+  // nearly as long as f16 ones at half the bytes (Qwen2.5-7B, 1024 72 / 69;
+  // TinyLlama, 1024 53 / 42). Partitions of up to three parts gain only from
+  // the work-groups of one wave (Llama-3-8B f16, 480 19.0 / 16.4, 896 15 / 20;
+  // Qwen2.5-7B q8_0, 1024 26 / 28).
+  int64_t limit = 5 * (int64_t)cu_count / 2;
+  if (subs < 4) limit = 2 * (int64_t)cu_count;
+  else if (elem == 1 && !pairs) limit = 4 * (int64_t)cu_count;
+  else if (elem == 1 || head_dim == 64) limit = 3 * (int64_t)cu_count;
+  if (waves > limit) return 0;
+  const int64_t bytes = n * n_kv_heads * group * max_parts * subs * (head_dim + 2) * 4;
+  return bytes > (int64_t)kPartsBytes ? 0 : (int)subs;
+}
+
+// Waves per work-group of the matrix-core decode kernel: four consecutive
+// waves of the grid, i.e. the kv-head groups of one (query, partition) item
+// on one CU, which then reads whole pool rows together (each wave still
+// streams its own item; bit-identical results). Measured against one wave
+// per work-group: the Llama-3-8B fused decode step 140.9 -> 137.9 us (the
+// kernel ~134 us in the plain, graph and fused passes alike instead of
+// 133-137), q8_0 decode 3.5% and the Qwen2.5-7B step 2% faster, 32 x 32k
+// decode within the noise, config 3's per-query pass 1.4% slower. The wave
+// index is made scalar (readfirstlane) and the grid index kept 32-bit: as a
+// vector value or a 64-bit division it cost SGPR spills and 10%.
+constexpr int kDecodeWaves = 4;
+
+// Launches of one wave per part take work-groups of one wave up to four a CU,
+// so that few waves spread over the CUs (one Llama-3-8B query of 5003 tokens:
+// 14.4 us against 17.5 with four waves a work-group); beyond, fewer
+// work-groups to dispatch.
+inline int decode_group_waves(bool fine, int64_t waves, int cu_count) {
+  return fine && waves <= 4 * (int64_t)cu_count ? 1 : kDecodeWaves;
+}
+
+// Work-groups of a launch: whole ones, so the last may hold waves past the
+// last item (decode_wave_item).
+inline unsigned decode_grid(int64_t waves, int group_waves) {
+  return (unsigned)((waves + group_waves - 1) / group_waves);
+}
+
+// The query (of n) and the index in it that a head group's wave takes in
+// query order, per_query waves a query; false: the wave has none.
+__host__ __device__ inline bool decode_wave_item(uint32_t wave, uint32_t per_query, int64_t n, int64_t &query,
+                                                 int &index) {
+  index = (int)(wave % per_query);
+  query = wave / per_query;
+  return query < n;
+}
+
 // Untuned f16 shapes on the matrix cores (attn_wide_kernel), and the parts per
 // query of a launch (AttnArgs::wide_parts): 0 where the states of n queries'
 // parts exceed kPartsBytes.

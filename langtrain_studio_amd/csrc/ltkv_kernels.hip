@@ -2092,24 +2092,13 @@ __device__ __forceinline__ h8 i8x8_to_h8_biased(const u32x2 &w) {
   return __builtin_bit_cast(h8, r);
 }
 
-// Waves per work-group of the matrix-core decode kernel: four consecutive
-// waves of the grid, i.e. the kv-head groups of one (query, partition) item
-// on one CU, which then reads whole pool rows together (each wave still
-// streams its own item; bit-identical results). Measured against one wave
-// per work-group: the Llama-3-8B fused decode step 140.9 -> 137.9 us (the
-// kernel ~134 us in the plain, graph and fused passes alike instead of
-// 133-137), q8_0 decode 3.5% and the Qwen2.5-7B step 2% faster, 32 x 32k
-// decode within the noise, config 3's per-query pass 1.4% slower. The wave
-// index is made scalar (readfirstlane) and the grid index kept 32-bit: as a
-// vector value or a 64-bit division it cost SGPR spills and 10%.
-constexpr int kDecodeWaves = 4;
-
-// FINE: one wave (a work-group of its own) per part of a partition, in
-// query order, its state written for attn_merge_subs_kernel. For launches
-// whose partitions would leave most of the chip idle: a wave streams a
-// 16-token tile of a Llama-3-8B pair of heads (16 KB) in ~1.1 us and one CU
-// takes in ~56 GB/s at most, so a partition of 1024 tokens lasts ~75 us
-// however idle the chip is, and four waves of one CU share that rate.
+// FINE: one wave per part of a partition, in query order (work-groups of one
+// wave or of kDecodeWaves: decode_group_waves), its state written for
+// attn_merge_subs_kernel. For launches whose partitions would leave most of
+// the chip idle: a wave streams a 16-token tile of a Llama-3-8B pair of heads
+// (16 KB) in ~1.1 us and one CU takes in ~56 GB/s at most, so a partition of
+// 1024 tokens lasts ~75 us however idle the chip is, and four waves of one CU
+// share that rate.
 template <typename T, int HD, int G, int NH, bool RUNS, bool FINE>
 __global__ void __launch_bounds__(64 * kDecodeWaves, NH == 1 && HD == 64 ? 4 : 1)
 attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const float *__restrict__ q,
@@ -2354,10 +2343,10 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
       qx = __builtin_amdgcn_readfirstlane((int)qx);
       part = __builtin_amdgcn_readfirstlane(part);
     } else {
-      const uint32_t per_query = (uint32_t)max_parts * (FINE ? (uint32_t)subs : 1u);
-      part = (int)((uint32_t)wave_idx % per_query);
-      qx = (uint32_t)wave_idx / per_query;
-      if (!FINE && qx >= n_queries) return;  // waves past the grid's last item
+      // (waves past the grid's last item leave before they load anything)
+      if (!decode_wave_item((uint32_t)wave_idx, (uint32_t)max_parts * (FINE ? (uint32_t)subs : 1u), n_queries, qx,
+                            part))
+        return;
     }
     const int64_t qi = qmap ? qmap[qx] : qx;
     int64_t len;
@@ -2987,11 +2976,8 @@ inline bool decode_ordered(const AttnArgs &a) {
 template <typename T, int HD, int G, int NH, bool RUNS, bool FINE = false>
 hipError_t launch_attn_mfma_k(const PoolGeom &g, const AttnArgs &a, int slots, int pair_items, hipStream_t s) {
   const int64_t waves = a.n * (a.n_kv_heads / NH) * a.max_parts * (FINE ? a.subs : 1);
-  // FINE work-groups of one wave up to four a CU, so that few waves spread
-  // over the CUs (one Llama-3-8B query of 5003 tokens: 14.4 us against 17.5
-  // with four waves a work-group); beyond, fewer work-groups to dispatch.
-  const int nw = FINE && waves <= 4 * (int64_t)a.cu_count ? 1 : kDecodeWaves;
-  const unsigned grid = (unsigned)((waves + nw - 1) / nw);
+  const int nw = decode_group_waves(FINE, waves, a.cu_count);
+  const unsigned grid = decode_grid(waves, nw);
   attn_mfma_kernel<T, HD, G, NH, RUNS, FINE><<<grid, 64 * nw, 0, s>>>(
       static_cast<const T *>(a.k_layer), static_cast<const T *>(a.v_layer), a.q, a.tables, a.table_stride,
       a.lens, a.out, a.part_o, a.part_ml, a.n_kv_heads, g.n_blocks, g.block_stride, g.slot_stride,
@@ -4548,11 +4534,6 @@ AttnWorkspace attention_workspace(int64_t n, int n_heads, int head_dim, int max_
   return w;
 }
 
-bool attention_tuned(int elem, int head_dim, int group) {
-  return (elem == 1 || elem == 2 || elem == 4) && (head_dim == 64 || head_dim == 128) && group >= 1 &&
-         group <= 8;
-}
-
 bool attention_supported(int elem, int head_dim, int group) {
   return (elem == 1 || elem == 2 || elem == 4) && head_dim >= 1 && head_dim <= kAnyMaxHeadDim && group >= 1;
 }
@@ -4642,31 +4623,6 @@ int attention_part_policy(int elem, int group, int n_kv_heads, bool valu) {
   (void)group;
   (void)n_kv_heads;
   return !valu && elem == 2 ? kPartCap : 0;
-}
-
-int attention_subs(int elem, int head_dim, int group, int n_kv_heads, bool valu, int64_t n, int max_parts,
-                   int max_part, int cu_count) {
-  if (elem == 4 || valu || !attention_tuned(elem, head_dim, group)) return 0;
-  const bool pairs = group <= 4 && n_kv_heads % 2 == 0;  // two kv heads a wave
-  const int64_t waves = n * (n_kv_heads / (pairs ? 2 : 1)) * max_parts;
-  const int64_t subs = div_up_tokens(max_part, sub_tokens(0, head_dim));
-  // Where the partitions number about half the SIMDs or less. Measured (us,
-  // partitions against parts; the lines lie between the last gain and the
-  // first loss): Llama-3-8B f16, 16 queries of 200-3000 tokens 80.5 / 32.2,
-  // 512 partitions 92-103 / 82, 616 of ragged lengths 90 / 64, 768 104 / 121;
-  // q8_0, 768 54 / 47, 1024 56 / 58. head_dim 64: SmolLM2 f16, 768 42 / 34;
-  // TinyLlama f16, 768 38 / 35, 1024 41 / 45. q8_0 waves of one head last
-  // nearly as long as f16 ones at half the bytes (Qwen2.5-7B, 1024 72 / 69;
-  // TinyLlama, 1024 53 / 42). Partitions of up to three parts gain only from
-  // the work-groups of one wave (Llama-3-8B f16, 480 19.0 / 16.4, 896 15 / 20;
-  // Qwen2.5-7B q8_0, 1024 26 / 28).
-  int64_t limit = 5 * (int64_t)cu_count / 2;
-  if (subs < 4) limit = 2 * (int64_t)cu_count;
-  else if (elem == 1 && !pairs) limit = 4 * (int64_t)cu_count;
-  else if (elem == 1 || head_dim == 64) limit = 3 * (int64_t)cu_count;
-  if (waves > limit) return 0;
-  const int64_t bytes = n * n_kv_heads * group * max_parts * subs * (head_dim + 2) * 4;
-  return bytes > (int64_t)kPartsBytes ? 0 : (int)subs;
 }
 
 int mq_rows(int, int) { return 32 * kMqWaves; }

@@ -102,3 +102,56 @@ def test_parts_under_capture_and_growth(gpu):
             want = g.decode_attention(0, q[pick].contiguous(), dt[pick].contiguous(), dl[pick].contiguous(), 32, 128)
             stream.synchronize()
             assert torch.equal(got.view(torch.int32), want[:2].view(torch.int32))
+
+
+# Fixed partitions whose launches end in the middle of a four-wave work-group
+# (1, 2 or 3 waves past the last item; head groups of 1, 2 and 3).
+@pytest.mark.parametrize("dtype,n_heads,n_kv,hd,part,n,longest", [
+    ("f16", 8, 1, 128, 640, 41, 3200),     # 1025 waves
+    ("f16", 9, 3, 64, 768, 23, 3200),      # 1035
+    ("f16", 14, 2, 64, 576, 57, 1600),     # 1026
+    ("f16", 24, 6, 128, 320, 23, 1600),    # 1035, two kv heads a wave
+    ("q8_0", 8, 1, 128, 320, 69, 1600),    # 1035
+    ("q8_0", 24, 6, 128, 1088, 13, 3200),  # 1170, partitions cut in two
+])
+def test_waves_past_the_last_part(gpu, dtype, n_heads, n_kv, hd, part, n, longest):
+    """The append fused into the launch, the plain launch and a plan, against
+    the same queries in a launch of whole partitions (bit-equal; query 0's
+    states lie behind the last slot of the partials) and the pools of a cache
+    that was written row by row."""
+    import torch
+
+    from langtrain_studio_amd import KvCache
+    from oracle import OracleKv
+
+    print(f"past the last part {dtype} {n_heads}/{n_kv}/{hd} {part} x {n}", flush=True)
+    rng = np.random.default_rng(part + n)
+    kvd = n_kv * hd
+    lens = [longest] + [int(x) for x in rng.integers(1, longest + 1, n - 1)]
+    blocks = sum(-(-x // BLOCK) for x in lens) + 4
+    order = rng.permutation(blocks)
+    g, o = KvCache(1, kvd, blocks * BLOCK, dtype=dtype, device=0), OracleKv(1, kvd, blocks * BLOCK, dtype=dtype)
+    g.set_attention_partition(part)
+    g.init_free_order(order)
+    o.init_free_order(order)
+    fill_sequences([("gpu", g), ("oracle", o)], {s: x - 1 for s, x in enumerate(lens)}, rng, kvd)
+    seqs, pos = np.arange(n, dtype=np.uint32), np.array(lens, np.uint64) - 1
+    sm = g.append_batch(seqs, pos)
+    np.testing.assert_array_equal(sm, o.append_batch(seqs, pos))
+    k, v = (rng.standard_normal((n, kvd), dtype=np.float32) for _ in range(2))
+    q = rng.standard_normal((n, n_heads * hd), dtype=np.float32)
+    tables, la = tables_and_lens(g, list(range(n)), lens)
+    dsm, dk, dv, dq, dt, dl = (torch.from_numpy(np.ascontiguousarray(x)).to(gpu) for x in (sm, k, v, q, tables, la))
+    fused = g.append_decode_attention(0, dsm, dk, dv, dq, dt, dl, n_heads, hd).cpu().numpy()
+    o.write_batch(0, sm, k, v)
+    for got, want in zip(g.read_pool(0), o.pool(0)):
+        np.testing.assert_array_equal(got, want)
+    pick = np.arange(n * 24) % n
+    whole = g.decode_attention(0, dq[pick].contiguous(), dt[pick].contiguous(), dl[pick].contiguous(), n_heads,
+                               hd).cpu().numpy()[:n]
+    plain = g.decode_attention(0, dq, dt, dl, n_heads, hd).cpu().numpy()
+    g.plan_attention(seqs, np.array(lens, np.uint32), n_heads, hd)
+    planned = g.planned_attention(0, dq).cpu().numpy()
+    for got in (fused, plain, planned):
+        np.testing.assert_array_equal(got.view(np.uint32), whole.view(np.uint32))
+    attention_close(whole, o.attention_tables(0, tables, la, q, n_heads, hd, threads=8), dtype)
