@@ -3902,6 +3902,15 @@ attn_any_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const 
 // and P as operands of their own, so that all 16 columns hold query heads:
 //   S^T[token][head] = K Q^T    A = K rows, loaded straight in the A layout
 //   O^T[d][head]    += V^T P^T  A = V^T through LDS and ds_read_b64_tr_b16
+// The split keeps f32 accuracy at any magnitude: every head of Q enters scaled
+// by the power of two that brings its largest element to [2^14, 2^15), and the
+// softmax reference lies kWideDrop below the maximum it was raised to, so the
+// largest weights are 2^7 to 2^15 and a lo part's quantum, 2^-24, is 2^-31 of
+// them or less. (With heads below 65504 unscaled and weights from 2^0, a head of
+// |q scale log2 e| ~ 1e-4 on K of ~1e3 had score errors of order 1e-4, 1e-6 in
+// f32.) A nonzero value whose hi part would be zero takes the smallest one,
+// 2^-24, which its lo part takes off again: an infinite K or V element then
+// stays an infinity under the smallest Q element or weight, as in f32.
 // The lo products take K and V with non-finite elements clamped: an infinite
 // element times a lo part of the other sign would turn an infinity (or a
 // weight of zero) of the f32 computation into a NaN.
@@ -3912,6 +3921,7 @@ attn_any_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const 
 // fit the buffer).
 // ----------------------------------------------------------------------------
 constexpr int kWideWaves = 4;
+constexpr float kWideDrop = 7.f;  // log2: weights up to 2^(drop + slack) = 2^15, inside f16
 constexpr int kWideParts = 32;
 
 // Tokens per part: 16 parts up to 4096 tokens (of 128 tokens at least), 256
@@ -3977,7 +3987,11 @@ attn_wide_kernel(const _Float16 *__restrict__ kpool, const _Float16 *__restrict_
   const int64_t qh = qi * n_heads + (int64_t)kvh * group + head0 + (live_head ? lr : 0);
 
   // B operands: 8 consecutive d of k step ks at d = 32 ks + 8 lq, as hi and
-  // lo parts (heads past the f16 range scaled by 2^-e: q_range_exp).
+  // lo parts of x 2^-e, e from the head's largest element (at least -110, so
+  // that 2^e and 2^-e are normal; an infinity counts as the largest finite
+  // value); the scores are multiplied by 2^e. (Converted before the first
+  // tile's loads: after them, the fetched Q and a tile's registers together
+  // cost head_dim 96 and 160 a wave per SIMD, 32 queries of 160 113 -> 147 us.)
   h8 qhi[KS], qlo[KS];
   float x[KS][8], amax = 0.f;
 #pragma unroll
@@ -3995,15 +4009,19 @@ attn_wide_kernel(const _Float16 *__restrict__ kpool, const _Float16 *__restrict_
       amax = __builtin_fmaxf(amax, __builtin_fabsf(x[ks][e]));
     }
   }
-  const int qex = q_range_exp(rows_reduce<true>(amax));
+  amax = __builtin_fminf(rows_reduce<true>(amax), 3.40282347e38f);
+  const int qup = amax > 0.f ? __builtin_amdgcn_frexp_expf(amax) - 15 : 0;
+  const int qex = qup < -110 ? -110 : qup;
   const float qinv = __builtin_ldexpf(1.f, -qex), qmul = __builtin_ldexpf(1.f, qex);
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float y = x[ks][e] * qinv;
-      qhi[ks][e] = (_Float16)y;
-      qlo[ks][e] = (_Float16)(y - (float)qhi[ks][e]);
+      // (a NaN stays one in hi; the lo part of either is any finite value)
+      const _Float16 h = (_Float16)__builtin_copysignf(__builtin_elementwise_maximum(__builtin_fabsf(y), 0x1p-24f), y);
+      qhi[ks][e] = y != 0.f ? h : (_Float16)0.f;
+      qlo[ks][e] = (_Float16)__builtin_fmaxf(y - (float)qhi[ks][e], -32.f);
     }
 
   const int32_t *tab = table_of(tables, table_stride, rows, n_rows, qi);
@@ -4071,11 +4089,12 @@ attn_wide_kernel(const _Float16 *__restrict__ kpool, const _Float16 *__restrict_
     }
     const float lmax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(sc[0], sc[1]),
                                                      __builtin_elementwise_maximum(sc[2], sc[3]));
-    if (__builtin_amdgcn_ballot_w64(lmax > m_ref + kDecodeSlack)) {
+    if (__builtin_amdgcn_ballot_w64(lmax > m_ref + (kWideDrop + kDecodeSlack))) {
       const float mx = rows_reduce<true>(lmax);
-      if (mx > m_ref + kDecodeSlack) {
-        const float alpha = __builtin_amdgcn_exp2f(m_ref - mx);
-        m_ref = mx;
+      if (mx > m_ref + (kWideDrop + kDecodeSlack)) {
+        const float ref = mx - kWideDrop;
+        const float alpha = __builtin_amdgcn_exp2f(m_ref - ref);
+        m_ref = ref;
         l_run *= alpha;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
@@ -4087,7 +4106,8 @@ attn_wide_kernel(const _Float16 *__restrict__ kpool, const _Float16 *__restrict_
     for (int i = 0; i < 4; ++i) {
       const float p = __builtin_amdgcn_exp2f(sc[i] - off);
       l_run += p;
-      ph[i] = (_Float16)p;
+      const _Float16 h = (_Float16)p;
+      ph[i] = p > 0.f ? __builtin_elementwise_max(h, (_Float16)0x1p-24f) : h;
       pl[i] = (_Float16)(p - (float)ph[i]);
     }
 #pragma unroll
