@@ -2050,23 +2050,6 @@ __device__ __forceinline__ bool decode_order_find(int64_t t, int64_t n, int lane
 // lanes, else the hi part f16(x) (columns past the group are discarded, any
 // finite value does).
 //
-// q8_0 weights x = p d (d the token's V scale, f16): hi = f16(p d), then
-// f16(p d + c) with c = hi * lo_m2 (lo_m2 = -1 on lo lanes, 0 on the others,
-// one v_pk_mul_f16 per pair) is the lo part on lo lanes and hi on the others;
-// p d is exact inside v_fma_mix, so the lo part is f16(p d - hi).
-__device__ __forceinline__ h4 weight_parts_scaled(const float (&p)[4], const h4 &d, const h2 &lo_m2) {
-  h4 r;
-#pragma unroll
-  for (int i = 0; i < 4; i += 2) {
-    const h2 hi = h2{(_Float16)__builtin_fmaf(p[i], (float)d[i], 0.f),
-                     (_Float16)__builtin_fmaf(p[i + 1], (float)d[i + 1], 0.f)};
-    const h2 c = hi * lo_m2;
-    r[i] = (_Float16)__builtin_fmaf(p[i], (float)d[i], (float)c[0]);
-    r[i + 1] = (_Float16)__builtin_fmaf(p[i + 1], (float)d[i + 1], (float)c[1]);
-  }
-  return r;
-}
-
 // The parts of four f32 weights: lo_mult is -1 on lo lanes and 0 on the
 // others, in a register, so f16(fma(f16(x), lo_mult, x)) is either part, one
 // v_fma_mix on the packed hi parts per element.
@@ -2079,6 +2062,21 @@ __device__ __forceinline__ h4 weight_parts(const float (&x)[4], float lo_mult) {
   r[2] = (_Float16)__builtin_fmaf((float)h23[0], lo_mult, x[2]);
   r[3] = (_Float16)__builtin_fmaf((float)h23[1], lo_mult, x[3]);
   return r;
+}
+
+// The parts of q8_0 weights p d (d the token's V scale), as those of the f32
+// products. The product is kept from being folded into the conversions: hi
+// as one v_fma_mixlo_f16 of p and d rounds once, the hi lanes' part of the f32
+// product twice, and where the two differed the pair was one f16 step off
+// (about one in 2^14 weights: a head of 1900 tokens up to 4e-5 off).
+__device__ __forceinline__ h4 weight_parts_scaled(const float (&p)[4], const h4 &d, float lo_mult) {
+  float x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = p[i] * (float)d[i];
+    asm("" : "+v"(x[i]));
+  }
+  return weight_parts(x, lo_mult);
 }
 
 // Stored quants x 8 -> f16 x 8 of 1152 + x (exact; the bias is taken out
@@ -2221,8 +2219,6 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   const bool hi_lane = lr < NQ, lo_lane = lr >= 16 - NQ;
   float lo_mult = lo_lane ? -1.f : 0.f;  // weight_parts: opaque to the optimiser
   asm volatile("" : "+v"(lo_mult));
-  h2 lo_m2 = lo_lane ? h2{-1.f16, -1.f16} : h2{0.f16, 0.f16};  // weight_parts_scaled
-  asm volatile("" : "+v"(lo_m2));
   const int qj = hi_lane ? lr : (lo_lane ? 15 - lr : 0);  // the column's query head in the wave
   const int my_head = qj / G;                             // its kv head in the wave
   // The query operand is fetched (fetch_q) and converted (convert_q) apart:
@@ -2660,7 +2656,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
       h4 pw = pf;
       if constexpr (Q8) {
         const h4 d = *reinterpret_cast<const h4 *>(&ssc[1][(my_head * KS + g) * 16 + 4 * lq]);
-        pw = weight_parts_scaled(p, d, lo_m2);
+        pw = weight_parts_scaled(p, d, lo_mult);
       }
       h4 pb[NH];
 #pragma unroll

@@ -335,3 +335,51 @@ def test_q8_write_rope_bit_exact(gpu, n_heads, n_kv, head_dim, rope_dim, neox, b
     o.write_rope_batch(0, sm, p32, k, v, base, rope_dim, head_dim, neox, q=qo, n_heads=n_heads)
     np.testing.assert_array_equal(dq.cpu().numpy().view(np.uint32), qo.view(np.uint32))
     _assert_q8_equal(g, o, (0,))
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,lens", [
+    (28, 4, 128, [1143, 1861, 6511]),  # one kv head a wave, one wave per part
+    (32, 8, 128, [2277, 700] * 40),    # pairs of kv heads, whole partitions
+    (16, 4, 64, [1846, 3000, 500]),
+])
+def test_q8_weights_keep_f32_accuracy(gpu, n_heads, n_kv, hd, lens):
+    """Every head against 64-bit attention over the dequantised rows. The
+    scores are differences of f32 sums of up to ~1e3 (quants enter as 1152 + k),
+    good to a few 1e-6, the weights f32 products as f16 hi + lo pairs: 6e-6 at
+    most was measured. A pair whose hi parts round differently on its two lanes
+    is a whole f16 step of one weight off: 1.5e-5 to 4e-5 of a head of 2000
+    tokens, in a few heads of each launch."""
+    import torch
+
+    from langtrain_studio_amd import KvCache
+
+    print(f"q8_0 accuracy {n_heads}/{n_kv}/{hd}", flush=True)
+    rng = np.random.default_rng(hd + n_heads)
+    kvd, seqs = n_kv * hd, len(set(lens))
+    own = lens[:seqs]
+    blocks = sum(-(-x // BLOCK) for x in own)
+    g = KvCache(1, kvd, blocks * BLOCK, dtype="q8_0", device=0)
+    fill_sequences([("gpu", g)], dict(enumerate(own)), rng, kvd)
+    tables, _ = tables_and_lens(g, list(range(seqs)), own)
+    pick = np.arange(len(lens)) % seqs
+    q = rng.standard_normal((len(lens), n_heads * hd), dtype=np.float32)
+    got = g.decode_attention(0, *(torch.from_numpy(np.ascontiguousarray(x)).to(gpu) for x in (
+        q, tables[pick], np.array(lens, np.int32))), n_heads, hd).cpu().numpy().astype(np.float64)
+    rows = []
+    for quants, scales in zip(g.read_pool(0), g.read_scales(0)):
+        d = scales.view(np.float16).astype(np.float64).transpose(0, 2, 1)  # [block][slot][group]
+        rows.append((quants.astype(np.float64).reshape(blocks, BLOCK, -1, 32) * d[..., None]).reshape(blocks, BLOCK, kvd))
+    worst = 0.0
+    for i in range(min(len(lens), 6)):
+        s = pick[i]
+        k, v = (r[tables[s][:-(-lens[i] // BLOCK)]].reshape(-1, kvd)[:lens[i]] for r in rows)
+        for h in range(n_heads):
+            a = h // (n_heads // n_kv)
+            sc = (k[:, a * hd:(a + 1) * hd] @ q[i, h * hd:(h + 1) * hd].astype(np.float64)) * np.float64(
+                np.float32(1 / np.sqrt(hd)))
+            p = np.exp(sc - sc.max())
+            want = (p / p.sum()) @ v[:, a * hd:(a + 1) * hd]
+            err = np.linalg.norm(got[i, h * hd:(h + 1) * hd] - want) / np.linalg.norm(want)
+            worst = max(worst, err)
+    print(f"worst head {worst:.2e}", flush=True)
+    assert worst <= 1e-5
