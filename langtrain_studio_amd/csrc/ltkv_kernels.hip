@@ -1691,6 +1691,13 @@ __device__ __forceinline__ float rows_reduce(float x) {
 }
 
 constexpr float kDecodeSlack = 8.f;  // log2 headroom of the softmax reference
+// q8_0 weights enter their products times a V scale (~0.02 for rows of N(0, 1)),
+// so the lo parts of most are subnormal, multiples of 2^-24. Their reference lies
+// kQ8Drop below the maximum it was raised to and has that much less headroom:
+// the largest weights stay 2^8 (times a scale they must stay inside f16) and the
+// others gain four bits. Worst head of 28 / 4 / 128, 1143-6511 tokens, against
+// 64 bits: 6.0e-6 with the reference at the maximum, 2.0e-6 so; time unchanged.
+constexpr float kQ8Drop = 4.f;
 
 // ----------------------------------------------------------------------------
 // Parts of a partition. The matrix-core decode kernel sums each partition in
@@ -2627,11 +2634,12 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
     if (__builtin_amdgcn_ballot_w64(lmax > m_thr)) {
       const float mx = rows_reduce<true>(lmax);
       if (mx > m_thr) {
-        const float alpha = __builtin_amdgcn_exp2f(m_ref - mx);
+        const float ref = Q8 ? mx - kQ8Drop : mx;
+        const float alpha = __builtin_amdgcn_exp2f(m_ref - ref);
         const bool held = m_ref != -INFINITY;  // else the column's accumulators are still empty
-        m_ref = mx;
-        m_thr = mx + kDecodeSlack;
-        m_off = mx;
+        m_ref = ref;
+        m_thr = ref + kDecodeSlack;
+        m_off = ref;
         if (__builtin_amdgcn_ballot_w64(held)) {
           l_run *= alpha;
 #pragma unroll

@@ -345,7 +345,7 @@ def test_q8_write_rope_bit_exact(gpu, n_heads, n_kv, head_dim, rope_dim, neox, b
 def test_q8_weights_keep_f32_accuracy(gpu, n_heads, n_kv, hd, lens):
     """Every head against 64-bit attention over the dequantised rows. The
     scores are differences of f32 sums of up to ~1e3 (quants enter as 1152 + k),
-    good to a few 1e-6, the weights f32 products as f16 hi + lo pairs: 6e-6 at
+    good to a few 1e-6, the weights f32 products as f16 hi + lo pairs: 2e-6 at
     most was measured. A pair whose hi parts round differently on its two lanes
     is a whole f16 step of one weight off: 1.5e-5 to 4e-5 of a head of 2000
     tokens, in a few heads of each launch."""
@@ -382,4 +382,4 @@ def test_q8_weights_keep_f32_accuracy(gpu, n_heads, n_kv, hd, lens):
             err = np.linalg.norm(got[i, h * hd:(h + 1) * hd] - want) / np.linalg.norm(want)
             worst = max(worst, err)
     print(f"worst head {worst:.2e}", flush=True)
-    assert worst <= 1e-5
+    assert worst <= 5e-6
