@@ -83,7 +83,12 @@ LTKV_API const char *ltkv_last_error(void);
  * blocks, zero-filled K and V pools on HIP device `device` (or none for
  * LTKV_NO_DEVICE), free stack (0..n_blocks).rev(). Any kv_dim >= 1 (Q8_0:
  * a multiple of 32); rows whose byte length is a multiple of 16 take the
- * vectorised kernels, others element-wise ones. */
+ * vectorised kernels, others element-wise ones.
+ * A device cache also holds memory for attention partials (ltkv_bytes does
+ * not count it): a quarter of one layer's rows, at least 1 and at most 16
+ * MiB, from its creation (none if the device has no room left beside the
+ * pools); 32 MiB more from the first small launch that it does not suffice
+ * for; and a workspace for larger launches, grown on demand. */
 LTKV_API int ltkv_create(size_t n_layers, size_t kv_dim, size_t n_tokens, int dtype, int device,
                 ltkv_cache **out);
 LTKV_API void ltkv_destroy(ltkv_cache *c);
@@ -239,9 +244,9 @@ LTKV_API int ltkv_decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t
  * static device array of LTKV_NOALLOC_SCRATCH_BYTES on each device (held
  * until the process ends) instead of the cache's workspace, which
  * ltkv_decode_attention grows with hipMalloc on demand. (Launches small
- * enough to run one wave per part of a partition keep their partials in a
- * 64 MiB buffer that every device cache holds from its creation, on either
- * entry point.) A launch whose
+ * enough to run one wave per part of a partition keep their partials in
+ * memory the cache holds, see ltkv_create, and here in the scratch where that
+ * is too small.) A launch whose
  * partials need more fails with LTKV_ERR_ARG before anything is enqueued:
  * they take n * n_heads * P * (head_dim + 2) * 4 bytes, P counted for the
  * longest context the tables hold (T = table_stride * 16 tokens): 4 up to

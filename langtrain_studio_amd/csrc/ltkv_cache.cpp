@@ -145,9 +145,11 @@ struct ltkv_cache {
   // Attention workspace (partition partials), grown on demand.
   uint8_t *ws = nullptr;
   size_t ws_bytes = 0;
-  // Partials of small launches, held from creation: ltkv::kPartsBytes for the
-  // states of parts, as many for partition and group partials.
-  uint8_t *parts = nullptr;
+  // Memory for the partials of ordinary launches, held from creation
+  // (held_size), and the part states of launches that need more:
+  // ltkv::kPartsBytes, allocated by the first of those and then kept.
+  uint8_t *held = nullptr, *states = nullptr;
+  size_t held_bytes = 0;
   // The device's static scratch (ltkv_decode_attention_noalloc), looked up at
   // creation; shared by every cache on the device.
   uint8_t *scratch = nullptr;
@@ -424,18 +426,57 @@ int ensure_workspace(ltkv_cache *c, size_t bytes) {
   return LTKV_OK;
 }
 
-// Memory for a launch's partials: up to `limit` bytes (at most kPartsBytes) of
-// the buffer held from the cache's creation, after the parts' states (no
+// Bytes held from a cache's creation for launches' partials: a quarter of one
+// layer's K and V rows, which is about what the partitions of every sequence
+// take together (four per query; f16, 32 / 8 heads of 128, 64 tokens a
+// sequence: 67 KB of partials, 262 KB of rows), 1 to 16 MiB. (64 MiB whatever
+// the cache took ~150 us more to create, as any allocation of 2 MiB and more
+// does; smaller ones ~1 us.)
+size_t held_size(const ltkv_cache *c) {
+  const size_t quarter = c->layer_elems() * c->elem / 2;
+  return std::min<size_t>(std::max<size_t>(quarter, size_t{1} << 20), size_t{16} << 20);
+}
+
+// Memory for a launch's partition and group partials: the held memory (no
 // allocation on a first call; the launches of a cache follow each other on
-// its stream), the workspace beyond.
-int workspace(ltkv_cache *c, size_t bytes, size_t limit, uint8_t **base) {
-  if (bytes <= limit) {
-    *base = c->parts + ltkv::kPartsBytes;
+// its stream), the workspace where it is too small.
+int workspace(ltkv_cache *c, size_t bytes, uint8_t **base) {
+  if (bytes <= c->held_bytes) {
+    *base = c->held;
     return LTKV_OK;
   }
   if (int rc = ensure_workspace(c, bytes)) return rc;
   *base = c->ws;
   return LTKV_OK;
+}
+
+// Whether the cache's stream records its work (an error, e.g. the null stream
+// while another one records, counts as such).
+bool capturing(const ltkv_cache *c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+// Memory for `bytes` (at most kPartsBytes) of part states, `used` bytes of the
+// held memory being taken: the rest of it, or the cache's states buffer, or
+// with use_scratch (which allocates nothing) the device's scratch. Neither is
+// freed before the cache, so a captured launch's states stay where they are.
+// nullptr: none without an allocation that is not possible now (the launch then
+// runs without parts, with the same bits).
+uint8_t *part_states(ltkv_cache *c, size_t bytes, size_t used, bool use_scratch) {
+  static_assert(ltkv::kScratchBytes >= ltkv::kPartsBytes, "part states fit the scratch");
+  used = (used + 255) / 256 * 256;
+  if (used <= c->held_bytes && bytes <= c->held_bytes - used) return c->held + used;
+  if (!c->states && use_scratch) return c->scratch;
+  if (!c->states && !capturing(c) && hipMalloc((void **)&c->states, ltkv::kPartsBytes) != hipSuccess) {
+    (void)hipGetLastError();
+    c->states = nullptr;
+  }
+  return c->states;
 }
 
 // Uploads the resident-table changes made since the last call: only the
@@ -579,13 +620,28 @@ ltkv::AttnArgs attn_args(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, 
   return a;
 }
 
-// The part states of attn_wide_kernel's shapes go to the cache's parts buffer.
-void set_wide_parts(const ltkv_cache *c, ltkv::AttnArgs &a, size_t group, size_t max_len) {
+// Points a launch at memory for the states of its parts; without any it runs
+// one wave per partition (one work-group per query for attn_wide_kernel's
+// shapes).
+void set_parts(ltkv_cache *c, ltkv::AttnArgs &a, int subs, size_t used, bool use_scratch) {
+  const int parts = a.max_parts * subs;
+  const ltkv::AttnWorkspace ws = ltkv::attention_workspace(a.n, a.n_heads, a.head_dim, parts, true);
+  uint8_t *base = subs > 0 ? part_states(c, (size_t)ws.bytes, used, use_scratch) : nullptr;
+  if (!base) return;
+  a.subs = subs;
+  a.part_o = (float *)(base + ws.part_o_off);
+  a.part_ml = (float *)(base + ws.part_ml_off);
+}
+
+void set_wide_parts(ltkv_cache *c, ltkv::AttnArgs &a, size_t group, size_t max_len, bool use_scratch) {
   if (!ltkv::attention_wide((int)c->elem, a.head_dim, (int)group, a.valu)) return;
-  a.wide_parts = ltkv::attention_wide_parts(a.n, a.n_heads, a.head_dim, (int64_t)max_len);
-  const ltkv::AttnWorkspace ws = ltkv::attention_workspace(a.n, a.n_heads, a.head_dim, a.wide_parts, true);
-  a.part_o = (float *)(c->parts + ws.part_o_off);
-  a.part_ml = (float *)(c->parts + ws.part_ml_off);
+  const int parts = ltkv::attention_wide_parts(a.n, a.n_heads, a.head_dim, (int64_t)max_len);
+  const ltkv::AttnWorkspace ws = ltkv::attention_workspace(a.n, a.n_heads, a.head_dim, parts, true);
+  uint8_t *base = parts > 0 ? part_states(c, (size_t)ws.bytes, 0, use_scratch) : nullptr;
+  if (!base) return;
+  a.wide_parts = parts;
+  a.part_o = (float *)(base + ws.part_o_off);
+  a.part_ml = (float *)(base + ws.part_ml_off);
 }
 
 // Fewest shared full blocks and members for a prefix group.
@@ -1070,14 +1126,20 @@ int ltkv_create(size_t n_layers, size_t kv_dim, size_t n_tokens, int dtype, int 
     if ((e = hipMalloc((void **)&c->d_status, 4 * sizeof(int32_t))) != hipSuccess) rc = hip_fail(e, "hipMalloc(status)");
     else if ((e = hipMemset(c->d_status, 0, 4 * sizeof(int32_t))) != hipSuccess) rc = hip_fail(e, "hipMemset(status)");
   }
-  if (rc == LTKV_OK && (e = hipMalloc((void **)&c->parts, 2 * ltkv::kPartsBytes)) != hipSuccess)
-    rc = hip_fail(e, "hipMalloc(parts)");
   const size_t sbytes = c->q8() ? n_layers * c->layer_scales() * 2 : 0;
   if (rc == LTKV_OK && sbytes > 0) {
     if ((e = hipMalloc(&c->ks, sbytes)) != hipSuccess) rc = hip_fail(e, "hipMalloc(K scales)");
     else if ((e = hipMalloc(&c->vs, sbytes)) != hipSuccess) rc = hip_fail(e, "hipMalloc(V scales)");
     else if ((e = hipMemset(c->ks, 0, sbytes)) != hipSuccess) rc = hip_fail(e, "hipMemset(K scales)");
     else if ((e = hipMemset(c->vs, 0, sbytes)) != hipSuccess) rc = hip_fail(e, "hipMemset(V scales)");
+  }
+  if (rc == LTKV_OK) {  // where the pools leave no room, launches use the workspace
+    if (hipMalloc((void **)&c->held, held_size(c)) == hipSuccess) {
+      c->held_bytes = held_size(c);
+    } else {
+      (void)hipGetLastError();
+      c->held = nullptr;
+    }
   }
   if (rc == LTKV_OK && (e = hipEventCreateWithFlags(&c->pairs_done, hipEventDisableTiming)) != hipSuccess)
     rc = hip_fail(e, "hipEventCreate");
@@ -1103,7 +1165,8 @@ void ltkv_destroy(ltkv_cache *c) {
     if (c->d_order_counts) (void)hipFree(c->d_order_counts);
     if (c->d_order_pairs) (void)hipFree(c->d_order_pairs);
     if (c->ws) (void)hipFree(c->ws);
-    if (c->parts) (void)hipFree(c->parts);
+    if (c->held) (void)hipFree(c->held);
+    if (c->states) (void)hipFree(c->states);
     if (c->d_status) (void)hipFree(c->d_status);
     if (c->rope) (void)hipFree(c->rope);
     if (c->plan.done) (void)hipEventDestroy(c->plan.done);
@@ -1515,35 +1578,32 @@ int decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, size
   // Shapes outside the tuned kernels run the generic kernel over whole
   // contexts: no partition partials, so no workspace.
   const bool tuned = ltkv::attention_tuned((int)c->elem, (int)head_dim, (int)group);
-  // Small launches run one wave per part of a partition; the parts' states
-  // have a buffer of their own, so neither the workspace nor the scratch is
-  // needed, and the checks below stay those of one wave per partition.
-  const int subs = ltkv::attention_subs((int)c->elem, (int)head_dim, (int)group, (int)(c->kv_dim / head_dim), valu,
-                                        (int64_t)n, (int)max_parts,
-                                        ltkv::max_partition_size((int64_t)max_len, part, split), c->device_count_cu);
-  ltkv::AttnWorkspace ws =
+  const ltkv::AttnWorkspace ws =
       tuned ? ltkv::attention_workspace((int64_t)n, (int)n_heads, (int)head_dim, (int)max_parts)
             : ltkv::AttnWorkspace{0, 0, 0};
-  uint8_t *base = nullptr;
-  if (use_scratch) {
-    if ((size_t)ws.bytes > ltkv::kScratchBytes)
-      return fail(LTKV_ERR_ARG,
-                  "attention needs %lld bytes of partition partials, more than the %zu bytes of the "
-                  "no-allocation scratch",
-                  (long long)ws.bytes, ltkv::kScratchBytes);
-    base = c->scratch;
-  } else if (subs == 0) {
-    if (int rc = workspace(c, (size_t)ws.bytes, ltkv::kPartsBytes / 2, &base)) return rc;
-  }
-  if (subs > 0) {
-    ws = ltkv::attention_workspace((int64_t)n, (int)n_heads, (int)head_dim, (int)max_parts * subs, true);
-    base = c->parts;
-  }
-  ltkv::AttnArgs a = attn_args(c, layer, n, n_heads, head_dim, scale, d_q, d_out, ws, part,
-                               (int)max_parts, base);
+  if (use_scratch && (size_t)ws.bytes > ltkv::kScratchBytes)
+    return fail(LTKV_ERR_ARG,
+                "attention needs %lld bytes of partition partials, more than the %zu bytes of the "
+                "no-allocation scratch",
+                (long long)ws.bytes, ltkv::kScratchBytes);
+  ltkv::AttnArgs a = attn_args(c, layer, n, n_heads, head_dim, scale, d_q, d_out, ltkv::AttnWorkspace{}, part,
+                               (int)max_parts, nullptr);
   a.split = split;
-  a.subs = subs;
-  set_wide_parts(c, a, group, max_len);
+  // Small launches run one wave per part of a partition, whose states take the
+  // partials' place.
+  set_parts(c, a,
+            ltkv::attention_subs((int)c->elem, (int)head_dim, (int)group, a.n_kv_heads, valu, (int64_t)n,
+                                 (int)max_parts, ltkv::max_partition_size((int64_t)max_len, part, split),
+                                 c->device_count_cu),
+            0, use_scratch);
+  set_wide_parts(c, a, group, max_len, use_scratch);
+  if (a.subs == 0 && ws.bytes > 0) {
+    uint8_t *base = c->scratch;
+    if (!use_scratch)
+      if (int rc = workspace(c, (size_t)ws.bytes, &base)) return rc;
+    a.part_o = (float *)(base + ws.part_o_off);
+    a.part_ml = (float *)(base + ws.part_ml_off);
+  }
   a.tables = d_tables;
   a.table_stride = (int64_t)table_stride;
   a.rows = d_rows;
@@ -1784,13 +1844,15 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
   const size_t pre_o_off = ((size_t)ws.bytes + 255) / 256 * 256;
   const size_t pre_ml_off = pre_o_off + pre_slots * P.head_dim * 4;
   uint8_t *base = nullptr;
-  if (int rc = workspace(c, pre_ml_off + pre_slots * 2 * 4, ltkv::kPartsBytes, &base)) return rc;
+  const size_t ws_bytes = pre_ml_off + pre_slots * 2 * 4;
+  if (int rc = workspace(c, ws_bytes, &base)) return rc;
+  const size_t held_used = base == c->held ? ws_bytes : 0;
   const int32_t *d = reinterpret_cast<const int32_t *>(P.d);
   const ltkv::PoolGeom g = head_geom(c, P.head_dim);
   ltkv::AttnArgs a = attn_args(c, layer, P.n, P.n_heads, P.head_dim, scale, d_q, d_out, ws, part,
                                (int)max_parts, base);
   a.split = split;
-  set_wide_parts(c, a, group, P.sstride * LTKV_BLOCK);
+  set_wide_parts(c, a, group, P.sstride * LTKV_BLOCK, false);
   // Short remainders in one partition each and no group-only queries: the
   // decode kernel writes every output itself (folding group partials).
   a.merge_free = grouped && part > 0 && P.max_suffix <= (size_t)(part / split) && !P.empty_with_groups;
@@ -1834,16 +1896,12 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
   }
   // Small launches as decode_attention's.
   auto set_subs = [&](ltkv::AttnArgs &w) {
-    w.subs = ltkv::attention_subs((int)c->elem, (int)P.head_dim, (int)group, w.n_kv_heads, w.valu, w.n,
-                                  (int)max_parts,
-                                  ltkv::max_partition_size((int64_t)(P.sstride * LTKV_BLOCK), part, split),
-                                  c->device_count_cu);
-    if (w.subs > 0) {
-      const ltkv::AttnWorkspace pw =
-          ltkv::attention_workspace(w.n, w.n_heads, w.head_dim, (int)max_parts * w.subs, true);
-      w.part_o = (float *)(c->parts + pw.part_o_off);
-      w.part_ml = (float *)(c->parts + pw.part_ml_off);
-    }
+    set_parts(c, w,
+              ltkv::attention_subs((int)c->elem, (int)P.head_dim, (int)group, w.n_kv_heads, w.valu, w.n,
+                                   (int)max_parts,
+                                   ltkv::max_partition_size((int64_t)(P.sstride * LTKV_BLOCK), part, split),
+                                   c->device_count_cu),
+              held_used, false);
   };
   if (!grouped) {
     set_subs(a);

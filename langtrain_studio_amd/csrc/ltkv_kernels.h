@@ -252,8 +252,7 @@ int attention_split(int elem, int group, int n_kv_heads);
 int attention_part_policy(int elem, int group, int n_kv_heads, bool valu);
 // Parts per partition of a plain decode launch of n queries (AttnArgs::subs),
 // max_parts partitions of at most max_part tokens each; 0: one wave per
-// partition. Their states fit kPartsBytes (of a buffer each cache holds from
-// its creation, so no launch allocates for them).
+// partition. Their states fit kPartsBytes.
 constexpr size_t kPartsBytes = size_t{32} << 20;
 inline int attention_subs(int elem, int head_dim, int group, int n_kv_heads, bool valu, int64_t n, int max_parts,
                           int max_part, int cu_count) {

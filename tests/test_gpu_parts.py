@@ -155,3 +155,47 @@ def test_waves_past_the_last_part(gpu, dtype, n_heads, n_kv, hd, part, n, longes
     for got in (fused, plain, planned):
         np.testing.assert_array_equal(got.view(np.uint32), whole.view(np.uint32))
     attention_close(whole, o.attention_tables(0, tables, la, q, n_heads, hd, threads=8), dtype)
+
+
+def test_held_memory_follows_the_cache(gpu):
+    """A cache of one block holds little more than its pools. Part states that
+    its held memory is too small for (8 queries of 2000 tokens on one sequence:
+    2 129 920 bytes, 2 048 000 held) go to the scratch, to a buffer allocated once,
+    or, under capture on a cache that has none, nowhere: the launch runs whole
+    partitions. All with the same bits."""
+    import torch
+
+    from langtrain_studio_amd import KvCache
+
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info(gpu)[0]
+    small = KvCache(1, 1024, BLOCK, dtype="f32", device=0)
+    assert free - torch.cuda.mem_get_info(gpu)[0] < 16 << 20  # allocations come in steps of up to a few MiB
+    del small
+
+    rng = np.random.default_rng(12)
+    n, length = 8, 2000
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        g = KvCache(1, 1024, length, dtype="f16", device=0, stream=stream)
+        fill_sequences([("gpu", g)], {0: length}, rng, 1024)
+        tables, la = tables_and_lens(g, [0] * n, [length] * n)
+        dt, dl = torch.from_numpy(tables).to(gpu), torch.from_numpy(la).to(gpu)
+        q = torch.randn((n, 32 * 128), device=gpu)
+        out = torch.zeros_like(q)
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            g.decode_attention(0, q, dt, dl, 32, 128, out=out)
+        pick = np.arange(200) % n
+        whole = lambda: g.decode_attention(0, q[pick].contiguous(), dt[pick].contiguous(), dl[pick].contiguous(), 32,
+                                           128)[:n]
+        for _ in range(3):
+            q.normal_()
+            graph.replay()
+            got = [out.clone(), g.decode_attention(0, q, dt, dl, 32, 128, noalloc=True),
+                   g.decode_attention(0, q, dt, dl, 32, 128), g.decode_attention(0, q, dt, dl, 32, 128, noalloc=True)]
+            want = whole()
+            stream.synchronize()
+            for x in got:
+                assert torch.equal(x.view(torch.int32), want.view(torch.int32))
