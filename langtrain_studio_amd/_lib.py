@@ -97,3 +97,18 @@ def load() -> C.CDLL:
 
 def last_error() -> str:
     return load().ltkv_last_error().decode(errors="replace")
+
+
+def wait_event(event) -> None:
+    """Waits on the host for a torch.cuda.Event recorded outside any capture,
+    also while a stream records: HIP refuses the wait in the default capture
+    mode, so this thread's mode is relaxed for it. (The library's handle
+    resolves the call in the HIP runtime it is linked to.)"""
+    exchange = load().hipThreadExchangeStreamCaptureMode
+    mode = C.c_int(2)  # hipStreamCaptureModeRelaxed
+    if exchange(C.byref(mode)) != 0:
+        raise RuntimeError("hipThreadExchangeStreamCaptureMode failed")
+    try:
+        event.synchronize()
+    finally:
+        exchange(C.byref(mode))

@@ -18,6 +18,7 @@ from typing import Optional, Sequence
 
 import numpy as np
 
+from . import _lib
 from .kv import BLOCK, KvCache
 
 
@@ -163,7 +164,7 @@ class PagedKvBackend:
         already applied) into the claimed cells, then attention of q
         ([n][n_heads*head_dim] f32) over each token's sequence."""
         if plan.upload is not None and plan.upload[0] != self.kv._stream:  # the cache changed streams since
-            plan.upload[1].synchronize()
+            _lib.wait_event(plan.upload[1])
             plan.upload = None
         if plan.decode_only:  # ltkv_append_decode_attention: bit-identical to write + attention
             return self.kv.append_decode_attention(layer, plan.slot_mapping, k, v, q, plan.tables, plan.lens,

@@ -48,3 +48,38 @@ def test_steps_without_waiting(gpu, descriptor, case):
         return torch.stack(outs)
 
     assert torch.equal(run(True).view(torch.int32), run(False).view(torch.int32))
+
+
+@pytest.mark.parametrize("descriptor", ["tables", "resident", "planned"])
+def test_layers_captured_after_a_step_begins(gpu, descriptor):
+    """begin_step on one stream, the step's layers recorded on another: the
+    graph's replays give what the eager layers give."""
+    import torch
+
+    from langtrain_studio_amd.backend import BatchToken, PagedKvBackend
+
+    heads, n_kv, hd, n = 8, 2, 128, 5
+    own, side = torch.cuda.Stream(), torch.cuda.Stream()
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    q, k, v = (torch.randn((n, w), generator=gen, device="cuda") for w in (heads * hd, n_kv * hd, n_kv * hd))
+    out = torch.zeros((n, heads * hd), device="cuda")
+    torch.cuda.synchronize()
+    be = PagedKvBackend(1, heads, n_kv, hd, 64 * 16, n_seq_max=n, descriptor=descriptor, stream=own)
+    with torch.cuda.stream(own):
+        for t in range(3):
+            plan = be.begin_step([BatchToken(0, t, s) for s in range(n)])
+            be.layer(plan, 0, q, k, v)  # (sizes what is sized on demand)
+        plan = be.begin_step([BatchToken(0, 3, s) for s in range(n)])
+        be.kv.sync_tables()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        be.kv.set_stream(side)
+        be.layer(plan, 0, q, k, v, out=out)
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            q.normal_(generator=gen)
+            graph.replay()
+            got = out.clone()
+            want = be.layer(plan, 0, q, k, v)
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
