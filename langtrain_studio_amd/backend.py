@@ -131,9 +131,13 @@ class PagedKvBackend:
     def begin_step(self, batch: Sequence[BatchToken]) -> StepPlan:
         """Claim every token's cell (model.rs:380-383) and upload the step's
         slot mapping, block tables and lengths. Raises KvCacheFull /
-        NonContiguous like the reference's ``?``."""
+        NonContiguous like the reference's ``?``. Not inside a stream
+        capture: a replay would claim no cells, and its upload would read
+        staging that later steps rewrite."""
         import torch
 
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("begin_step cannot be captured: begin the step before the capture, capture its layers")
         if len(batch) > self._n_batch:
             raise ValueError(f"batch of {len(batch)} exceeds n_batch {self._n_batch}")
         seqs = np.array([b.seq for b in batch], dtype=np.uint32)

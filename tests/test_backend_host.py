@@ -39,3 +39,17 @@ def test_descriptor_is_checked():
         _meta(descriptor="bogus")
     with pytest.raises(ValueError):
         PagedKvBackend(1, 6, 4, 64, 64, device=None)  # 6 query heads over 4 kv heads
+
+
+def test_begin_step_is_refused_while_a_stream_records(monkeypatch):
+    """A step's upload must not be recorded: a replay would read staging that
+    later steps rewrite. Refused before any cell is claimed."""
+    import torch
+
+    from langtrain_studio_amd.backend import BatchToken
+
+    b = _meta()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="captured"):
+        b.begin_step([BatchToken(0, 0, 0)])
+    assert b.kv.len(0) == 0

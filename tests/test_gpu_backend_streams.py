@@ -53,7 +53,8 @@ def test_steps_without_waiting(gpu, descriptor, case):
 @pytest.mark.parametrize("descriptor", ["tables", "resident", "planned"])
 def test_layers_captured_after_a_step_begins(gpu, descriptor):
     """begin_step on one stream, the step's layers recorded on another: the
-    graph's replays give what the eager layers give."""
+    graph's replays give what the eager layers give. begin_step itself is
+    refused while the stream records, before it claims a cell."""
     import torch
 
     from langtrain_studio_amd.backend import BatchToken, PagedKvBackend
@@ -75,6 +76,9 @@ def test_layers_captured_after_a_step_begins(gpu, descriptor):
     with torch.cuda.graph(graph, stream=side):
         be.kv.set_stream(side)
         be.layer(plan, 0, q, k, v, out=out)
+        with pytest.raises(RuntimeError, match="captur"):
+            be.begin_step([BatchToken(0, 4, s) for s in range(n)])
+    assert be.kv.len(0) == 4
     for _ in range(3):
         with torch.cuda.stream(side):
             q.normal_(generator=gen)
