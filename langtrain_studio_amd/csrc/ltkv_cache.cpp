@@ -1856,6 +1856,7 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
   // Short remainders in one partition each and no group-only queries: the
   // decode kernel writes every output itself (folding group partials).
   a.merge_free = grouped && part > 0 && P.max_suffix <= (size_t)(part / split) && !P.empty_with_groups;
+  a.short_rest = grouped && P.max_suffix <= kShortRemainder;
   a.pass_empty = grouped && P.pass_empty;
   a.tables = d + P.off_stables;
   a.table_stride = (int64_t)P.sstride;
@@ -1914,7 +1915,7 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
     w.n = (int64_t)P.n_plain;
     w.qmap = d + P.off_qmap;
     w.pre_parts = nullptr;
-    w.merge_free = false;
+    w.merge_free = w.short_rest = false;
     set_subs(w);
     HIP_TRY(ltkv::launch_decode_attention(g, w, c->stream), "decode attention launch");
     if (P.n_pass == P.n_plain) return LTKV_OK;

@@ -134,6 +134,9 @@ struct AttnArgs {
   // partition, and none with group partials has an empty remainder (the
   // matrix-core kernel folds group partials of single-partition queries).
   bool merge_free;
+  // The caller knows that every query reads a short remainder after group
+  // partials (decode_ordered).
+  bool short_rest;
   // The caller knows the context kernel has nothing to do: every query has
   // group partials and an empty remainder, so only the merge runs (it folds
   // the group partials by itself).

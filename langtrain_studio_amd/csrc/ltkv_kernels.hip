@@ -2965,13 +2965,19 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   if (fault_q >= 0) report_fault(status, kFaultTable, fault_q);
 }
 
-// Launches of up to kOrderMaxQueries queries take their items longest first;
-// short remainders after group partials (merge_free: one partition each) keep
-// query order, where the scan would cost more than it gives. The 120 decodes
-// of 512-8191 tokens beside eight 512-token chunks (Qwen2.5-7B, one query map
-// entry each): 233 us in query order, 162 us so.
-inline bool decode_ordered(const AttnArgs &a) {
-  return !a.merge_free && a.n > 1 && a.n <= kOrderMaxQueries;
+// Launches of up to kOrderMaxQueries queries take their items longest first:
+// the 120 decodes of 512-8191 tokens beside eight 512-token chunks
+// (Qwen2.5-7B, one query map entry each) 233 us in query order, 162 us so.
+// Short remainders after group partials (short_rest) are nearly equal and pay
+// each wave's scan for little: in one partition each they keep query order,
+// and otherwise as long as all waves start at once (four a CU). Forks of 992
+// shared tokens, Llama-3-8B f16, us a step, query order / longest first: 5 of
+// 138 own tokens 26.4 / 27.1, 32 32.1 / 32.8, 128 (1024 waves) 50.9 / 50.1,
+// 128 of 488 73.9 / 75.5; 200 of 138 (1600 waves) 70.0 / 65.1, 200 of 488
+// 123.6 / 110.1.
+inline bool decode_ordered(const AttnArgs &a, int64_t waves) {
+  if (a.merge_free || a.n <= 1 || a.n > kOrderMaxQueries) return false;
+  return !a.short_rest || waves > 4 * (int64_t)a.cu_count;
 }
 
 // One wave per item (a partition of NH kv heads of one query), kDecodeWaves
@@ -2990,7 +2996,7 @@ hipError_t launch_attn_mfma_k(const PoolGeom &g, const AttnArgs &a, int slots, i
       a.max_len, a.pre_o, a.pre_ml, a.max_pre_parts, a.new_slots, a.new_k, a.new_v, a.new_stride,
       static_cast<T *>(const_cast<void *>(a.k_layer)), static_cast<T *>(const_cast<void *>(a.v_layer)),
       static_cast<uint16_t *>(const_cast<void *>(a.k_scale)), static_cast<uint16_t *>(const_cast<void *>(a.v_scale)), a.n,
-      decode_ordered(a) ? 1 : 0, slots, pair_items, a.subs, a.status);
+      decode_ordered(a, waves) ? 1 : 0, slots, pair_items, a.subs, a.status);
   if constexpr (FINE) return launch_merge_subs<HD>(a, s);
   return launch_merge<HD>(a, s, true);
 }
@@ -3014,7 +3020,8 @@ hipError_t launch_attn_mfma_t(const PoolGeom &g, const AttnArgs &a, hipStream_t 
       return blocks * nw;
     }();
     const int64_t slots = (int64_t)per_cu * a.cu_count;
-    if (decode_ordered(a) && slots > 0 && a.n * (a.n_kv_heads / NH) * a.max_parts >= 2 * slots)
+    const int64_t waves = a.n * (a.n_kv_heads / NH) * a.max_parts;
+    if (decode_ordered(a, waves) && slots > 0 && waves >= 2 * slots)
       return launch_attn_mfma_k<T, HD, G, NH, true>(g, a, (int)slots, 0, s);
   }
   // Work-groups per CU of the kernel without runs; with two, the items of
