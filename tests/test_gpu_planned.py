@@ -387,3 +387,15 @@ def test_q8_prefill_chunk_causal(gpu, n_heads, n_kv, head_dim, ctx, chunk):
     g, o, seqs, lens = _prefill_state(rng, n_kv * head_dim, [(0, ctx, chunk)], dtype="q8_0")
     stats, *_ = _run(gpu, g, o, seqs, lens, n_heads, head_dim, rng, dtype="q8_0")
     assert stats["groups"] == 1 and stats["grouped"] == chunk
+
+
+@pytest.mark.parametrize("n_heads,n_kv,head_dim", [(32, 4, 64), (32, 8, 128)])
+@pytest.mark.parametrize("tokens", [1100, 1400, 2100, 2400, 5000])
+def test_merge_of_range_partials(gpu, n_heads, n_kv, head_dim, tokens):
+    """A short chunk whose range is cut every 256 tokens or so: 4, 5, 8, 9 and
+    19 partials a query, i.e. the merge's loads up front and, past eight of
+    them, its loop."""
+    rng = np.random.default_rng(tokens + head_dim)
+    g, o, seqs, lens = _prefill_state(rng, n_kv * head_dim, [(0, tokens - 20, 20)])
+    stats, *_ = _run(gpu, g, o, seqs, lens, n_heads, head_dim, rng)
+    assert stats["groups"] == 1 and stats["grouped"] == 20
