@@ -2116,8 +2116,7 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
                  float *__restrict__ part_ml, int n_kv_heads, int64_t n_blocks, int64_t block_stride,
                  int64_t slot_stride, int64_t head_stride, float qscale, int part_tokens,
                  int split, int max_parts, const int32_t *__restrict__ pre_parts,
-                 const int32_t *__restrict__ qmap, const uint16_t *__restrict__ kscale,
-                 const uint16_t *__restrict__ vscale, const int32_t *__restrict__ rows, int64_t n_rows,
+                 const int32_t *__restrict__ qmap, const int32_t *__restrict__ rows, int64_t n_rows,
                  int64_t max_len, const float *__restrict__ pre_o, const float *__restrict__ pre_ml,
                  int max_pre_parts, const int32_t *__restrict__ new_slots,
                  const float *__restrict__ new_k, const float *__restrict__ new_v, int64_t new_stride,
@@ -2299,8 +2298,9 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   const int64_t sgroups = slot_stride >> 5;
   const int64_t shead = ((int64_t)kvh0 * head_stride >> 5) * 32;
   const int sidx = NSC <= 64 ? lane % NSC : 2 * lane;
-  // (q8_0: through the pointers that the fused append stores to, so that the
-  // tiles' loads stay after it)
+  // (q8_0: quants and scales through the pointers that the fused append stores
+  // to, kdst .. vsdst, and through no others, so that the tiles' loads stay
+  // after it)
   const char *kbase = reinterpret_cast<const char *>((Q8 ? kdst : kpool) + (int64_t)kvh0 * head_stride);
   const char *vbase = reinterpret_cast<const char *>((Q8 ? vdst : vpool) + (int64_t)kvh0 * head_stride);
   const int64_t block_bytes = block_stride * (int64_t)sizeof(T);
@@ -2996,8 +2996,7 @@ hipError_t launch_attn_mfma_k(const PoolGeom &g, const AttnArgs &a, int slots, i
       static_cast<const T *>(a.k_layer), static_cast<const T *>(a.v_layer), a.q, a.tables, a.table_stride,
       a.lens, a.out, a.part_o, a.part_ml, a.n_kv_heads, g.n_blocks, g.block_stride, g.slot_stride,
       g.head_stride, a.scale * kLog2e, a.part_tokens, a.split, a.max_parts, a.pre_parts, a.qmap,
-      static_cast<const uint16_t *>(a.k_scale), static_cast<const uint16_t *>(a.v_scale), a.rows, a.n_rows,
-      a.max_len, a.pre_o, a.pre_ml, a.max_pre_parts, a.new_slots, a.new_k, a.new_v, a.new_stride,
+      a.rows, a.n_rows, a.max_len, a.pre_o, a.pre_ml, a.max_pre_parts, a.new_slots, a.new_k, a.new_v, a.new_stride,
       static_cast<T *>(const_cast<void *>(a.k_layer)), static_cast<T *>(const_cast<void *>(a.v_layer)),
       static_cast<uint16_t *>(const_cast<void *>(a.k_scale)), static_cast<uint16_t *>(const_cast<void *>(a.v_scale)), a.n,
       decode_ordered(a, waves) ? 1 : 0, slots, pair_items, a.subs, a.status);
