@@ -223,15 +223,17 @@ LTKV_API int ltkv_gather(ltkv_cache *c, size_t layer, size_t n, const int32_t *d
  * d_tables[i*table_stride]; query head h uses kv head h/(n_heads/n_kv_heads).
  * Softmax of q.k*scale over the positions, times V; d_out is
  * [n][n_heads*head_dim] f32. Any group size and head_dim <= 1024: head_dim
- * 64 or 128 with groups of 1..8 take the tuned kernels, other shapes a
- * generic one (one work-group per query head, whole contexts).
+ * 64 or 128 with groups of 1..8 take the tuned kernels, other f16 shapes with
+ * head_dim a multiple of 8 up to 256 a matrix-core kernel of their own, the
+ * rest a generic one (one work-group per query head, whole contexts).
  * d_lens[i] == 0 yields zeros. A table entry outside the pool is read as
  * block 0 and reported by ltkv_synchronize (the reference panics, kv.rs:147).
  * Q may have any finite magnitude, as the reference's f32 scores allow
  * (model.rs:450,455-461): the matrix-core kernels (f16 and Q8_0 pools) take
  * q * scale * log2(e) as f16 hi + lo operands, and a query head whose
  * elements reach 65504 (|q| ~ 5.1e5 at head_dim 128) enters the products
- * scaled by 2^-e, its scores multiplied by 2^e afterwards (both exact). */
+ * scaled by 2^-e, its scores multiplied by 2^e afterwards (both exact; other
+ * f16 shapes scale every head so, small ones up). */
 LTKV_API int ltkv_decode_attention(ltkv_cache *c, size_t layer, size_t n, size_t n_heads, size_t head_dim,
                           float scale, const float *d_q, const int32_t *d_tables,
                           size_t table_stride, const int32_t *d_lens, float *d_out);

@@ -197,8 +197,8 @@ __host__ __device__ inline int split_partition(int64_t len, int part_tokens, int
   return split == 1 ? pt : (split == 2 ? pt >> 1 : pt / split);
 }
 
-// Tokens per part of a partition in the matrix-core decode kernel.
-// (32 KB of an f16 head's K and V rows up to 8192 tokens of context, more
+// Tokens per part of a partition in the matrix-core decode kernel (32 KB of an
+// f16 head's K rows and as much of V up to 8192 tokens of context, twice that
 // beyond): short enough that one short chat spreads over the chip, and fewer
 // parts where the partitions alone are many, since a wave that streams a
 // whole partition pays ~0.15 us per part for the fold. A function of the
@@ -263,7 +263,7 @@ inline int attention_subs(int elem, int head_dim, int group, int n_kv_heads, boo
   const bool pairs = group <= 4 && n_kv_heads % 2 == 0;  // two kv heads a wave
   const int64_t waves = n * (n_kv_heads / (pairs ? 2 : 1)) * max_parts;
   const int64_t subs = div_up_tokens(max_part, sub_tokens(0, head_dim));
-  // Where the partitions number about half the SIMDs or less. Measured (us,
+  // Up to 2 to 4 waves of one partition each a CU, by shape. Measured (us,
   // partitions against parts; the lines lie between the last gain and the
   // first loss): Llama-3-8B f16, 16 queries of 200-3000 tokens 80.5 / 32.2,
   // 512 partitions 92-103 / 82, 616 of ragged lengths 90 / 64, 768 104 / 121;

@@ -1634,8 +1634,9 @@ attn16_kernel(T *kpool, T *vpool, const float *__restrict__ q,
 // 32-element scale group is a k step of the score product, scaled after
 // it, and a separate P' (P times the V group scale) for the O tiles of the
 // group. The softmax reference per column is common to the four lane rows
-// and raised only when a score exceeds it by kDecodeSlack (ballot), so the
-// weights p = 2^(s - ref) <= 2^8 need no exchange on the fast path.
+// and raised only when a score exceeds it by kDecodeSlack (ballot; q8_0
+// references lie kQ8Drop below the maximum), so the weights
+// p = 2^(s - ref) <= 2^8 need no exchange on the fast path.
 // ----------------------------------------------------------------------------
 template <int B>
 struct BufVec;
@@ -2108,6 +2109,11 @@ __device__ __forceinline__ h8 i8x8_to_h8_biased(const u32x2 &w) {
 // (16 KB) in ~1.1 us and one CU takes in ~56 GB/s at most, so a partition of
 // 1024 tokens lasts ~75 us however idle the chip is, and four waves of one CU
 // share that rate.
+//
+// Launch bounds: one-head waves of head_dim 64 take 125 registers and run four
+// a SIMD; left to itself the compiler takes 129-132, and three (96 queries of
+// 1000-3000 tokens, f16: TinyLlama 48.2 us against 47.5, SmolLM2 41.6 / 39.9;
+// q8_0 within 1% either way).
 template <typename T, int HD, int G, int NH, bool RUNS, bool FINE>
 __global__ void __launch_bounds__(64 * kDecodeWaves, NH == 1 && HD == 64 ? 4 : 1)
 attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const float *__restrict__ q,
@@ -2155,8 +2161,8 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
   constexpr int VPITCH = HD * 2 + (!Q8 && HD == 128 ? 32 : 16);
   constexpr int NQ = NH * G;               // query heads of the wave
   constexpr int NSC = NH * KS * 16;        // q8_0 scale entries of a tile, K or V
-    // tiles in flight + 1 (FINE f16 pairs: two waves a SIMD with two, one with
-  // three: 16.1 against 14.4 us for one Llama-3-8B query of 5003 tokens)
+  // tiles in flight + 1 (FINE f16 pairs: two waves a SIMD with two, one with
+  // three: 14.4 against 16.1 us for one Llama-3-8B query of 5003 tokens)
   constexpr int STAGES = NH == 2 && (Q8 || (FINE && HD == 128)) ? 2 : 3;  // tiles in flight + 1
   using KV = typename BufVec<KB>::type;
   using SV = uint32_t;  // one or two b16 scale entries
@@ -2373,8 +2379,8 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
       // The query's parts come first in its index range, partition by
       // partition, so the waves past them are the range's end (with a fixed
       // number of waves per partition, the waves of parts that long contexts
-      // do not have fell on the same XCDs: one query of 32000 tokens 45.8
-      // us, 38 us so).
+      // do not have fell on the same XCDs: one query of 32000 tokens, with
+      // the merge, 45.8 us, 32 us so).
       const int per_part = div_up_tokens(pt, sub_tokens(len, HD));
       const int p = (int)((uint32_t)part / (uint32_t)per_part);
       sub = part - p * per_part;
@@ -3909,7 +3915,8 @@ attn_any_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const 
 // query heads, part of the context), and the parts (wide_part: a
 // function of the query's length) spread one query over the chip. Against attn_any_kernel, which reads a context once per query
 // head and one element per thread: 12 queries of 300-4000 tokens, 32 / 8
-// heads of 96, 1405 us -> 22 us (the launch's bytes: 13 us at 6.5 TB/s).
+// heads of 96, 1405 us -> 25 us, and 4 us of merge (the launch's bytes: 13 us
+// at 6.5 TB/s).
 //
 // Products as in attn_mfma_kernel, with HDP = head_dim padded to a template
 // width (columns past head_dim load as zeros) and the hi and lo parts of Q
@@ -3939,7 +3946,7 @@ constexpr float kWideDrop = 7.f;  // log2: weights up to 2^(drop + slack) = 2^15
 constexpr int kWideParts = 32;
 
 // Tokens per part: 16 parts up to 4096 tokens (of 128 tokens at least), 256
-// tokens up to 8192, 32 parts beyond. Listed launch above, us: 37 with 64
+// tokens up to 8192, 32 parts beyond. The launch above, us: 37 with 64
 // tokens at least and 32 parts, 31 so; 256 tokens at least cost one query of
 // 300 tokens, 8 heads of 256, 18 against 15.5 us, 16 parts beyond 4096 one of
 // 8000 tokens 25 against 22.

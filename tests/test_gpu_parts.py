@@ -1,6 +1,6 @@
 """Small decode launches run one wave per part of a partition
 (attention_subs) and merge the parts' states; larger ones stream whole
-partitions and fold the parts in registers. A query's bits must be the same
+partitions and fold the parts as they go. A query's bits must be the same
 either way, at the edges of the parts (128 or 256 tokens, twice that past
 8192), of the partitions and of a 16-token tile, through every entry point,
 and within the attention tolerance of the oracle."""
@@ -73,7 +73,7 @@ def test_parts_match_whole_partitions(gpu, dtype, n_heads, n_kv, hd, lens):
 
 
 def test_parts_under_capture_and_growth(gpu):
-    """The parts' buffer exists from the cache's creation: a small launch is
+    """The states' memory is held from the cache's creation: a small launch is
     captured on a cache that has run nothing, and the graph's replays stay
     right after larger launches have replaced the workspace."""
     import torch

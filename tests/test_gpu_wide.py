@@ -1,9 +1,11 @@
 """Decode attention on f16 pools of shapes outside head_dim 64 / 128 and
 groups of up to 8 (attn_wide_kernel): against the oracle at the edges of a
-tile (16 tokens), of the four waves' tiles (64), of the parts (32 a query,
-tokens up to 8192, 32 a query beyond) and of the padded widths, alone and in a batch with the
-same bits; a launch whose part states do not fit their buffer streams whole
-contexts, with the same bits; elements beyond f16 stay infinities."""
+tile (16 tokens), of the four waves' tiles (64), of the parts (a sixteenth of
+a query up to 4096 tokens, 128 at least, 256 tokens up to 8192, 32 a query
+beyond) and of the padded widths, alone and in a batch with the same bits; a
+launch whose part states exceed 32 MiB streams whole contexts, with the same
+bits; elements beyond f16 stay infinities, under any weight; Q of any
+magnitude keeps f32 accuracy."""
 
 from __future__ import annotations
 
