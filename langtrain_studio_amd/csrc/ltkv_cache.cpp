@@ -1781,6 +1781,53 @@ int ltkv_table_uploads(const ltkv_cache *c, uint64_t *entries) {
   return LTKV_OK;
 }
 
+namespace {
+
+// What the current plan's launches take: partition size and count, and the
+// partials' offsets and bytes.
+struct PlanShape {
+  int part, split;
+  size_t max_parts;
+  bool too_large;  // grid beyond one launch
+  ltkv::AttnWorkspace ws;
+  size_t pre_o_off, pre_ml_off, bytes;
+};
+
+PlanShape plan_shape(const ltkv_cache *c) {
+  const AttnPlan &P = c->plan;
+  const int n_kv = (int)(c->kv_dim / P.head_dim);
+  const int group = (int)P.n_heads / n_kv;
+  const bool grouped = P.groups > 0;
+  PlanShape L{};
+  // Grouped plans are batch-dependent anyway: when every query's remainder is
+  // short (forks reading a few private blocks), their per-query pass takes
+  // the plan's partition unless one is fixed; long remainders keep the
+  // per-query policy.
+  // Such remainders are not cut further (the q8_0 decode cut): a remainder in
+  // one partition lets its wave fold the group partials itself, with no merge
+  // launch (q8_0 config-3 step: the merge took ~11 us of ~98).
+  L.part = (int)c->attn_part_tokens;
+  const bool short_rem = grouped && L.part == 0 && P.sstride * LTKV_BLOCK <= kShortRemainder;
+  if (short_rem) L.part = P.suffix_part;
+  else if (L.part == 0)
+    L.part = ltkv::attention_part_policy((int)c->elem, group, n_kv,
+                                         c->attn_engine == LTKV_ENGINE_VALU && c->elem == 2);
+  L.split = short_rem ? 1 : ltkv::attention_split((int)c->elem, group, n_kv);
+  L.max_parts = (size_t)ltkv::max_partitions((int64_t)(P.sstride * LTKV_BLOCK), L.part) * L.split;
+  L.too_large = (uint64_t)P.n * n_kv * L.max_parts * 256 >= (1ull << 32);
+  // (no partition partials where the groups cover every query's context)
+  const bool covered = grouped && (P.pass_empty || P.groups_only);
+  if (!covered)
+    L.ws = ltkv::attention_workspace((int64_t)P.n, (int)P.n_heads, (int)P.head_dim, (int)L.max_parts, grouped);
+  const size_t pre_slots = grouped ? P.n * P.n_heads * (size_t)P.max_pre_parts : 0;
+  L.pre_o_off = ((size_t)L.ws.bytes + 255) / 256 * 256;
+  L.pre_ml_off = L.pre_o_off + pre_slots * P.head_dim * 4;
+  L.bytes = L.pre_ml_off + pre_slots * 2 * 4;
+  return L;
+}
+
+}  // namespace
+
 int ltkv_plan_attention(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *lens,
                         size_t n_heads, size_t head_dim, unsigned flags) {
   if (!c) return fail(LTKV_ERR_ARG, "cache is null");
@@ -1795,6 +1842,16 @@ int ltkv_plan_attention(ltkv_cache *c, size_t n, const uint32_t *seqs, const uin
   c->plan.f16_products = (flags & LTKV_PLAN_F16_PRODUCTS) != 0;
   if (c->device != LTKV_NO_DEVICE) {
     if (int rc = upload_plan(c)) return rc;
+    // The partials' memory while it can be had, so that the plan's launches can
+    // be captured on a cache that has run none (they allocate what is missing).
+    DeviceGuard dg(c->device);
+    uint8_t *base = nullptr;
+    if (n > 0 && dg.ok) {
+      const PlanShape L = plan_shape(c);
+      if (!L.too_large && L.bytes > c->held_bytes && L.bytes > c->ws_bytes && !capturing(c) &&
+          workspace(c, L.bytes, &base) != LTKV_OK)
+        (void)hipGetLastError();
+    }
   }
   c->plan.valid = true;
   c->plan.gen = c->gen;
@@ -1814,42 +1871,19 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
   if (((uintptr_t)d_q) % 16 != 0) return fail(LTKV_ERR_ARG, "q must be 16-byte aligned");
   const size_t group = P.n_heads / (c->kv_dim / P.head_dim);
   const bool grouped = P.groups > 0;
-  // Grouped plans are batch-dependent anyway: when every query's remainder is
-  // short (forks reading a few private blocks), their per-query pass takes
-  // the plan's partition unless one is fixed; long remainders keep the
-  // per-query policy.
-  // Such remainders are not cut further (the q8_0 decode cut): a remainder in
-  // one partition lets its wave fold the group partials itself, with no merge
-  // launch (q8_0 config-3 step: the merge took ~11 us of ~98).
-  int part = (int)c->attn_part_tokens;
-  const bool short_rem = grouped && part == 0 && P.sstride * LTKV_BLOCK <= kShortRemainder;
-  if (short_rem) part = P.suffix_part;
-  else if (part == 0)
-    part = ltkv::attention_part_policy((int)c->elem, (int)group, (int)(c->kv_dim / P.head_dim),
-                                       c->attn_engine == LTKV_ENGINE_VALU && c->elem == 2);
-  const int parts = ltkv::max_partitions((int64_t)(P.sstride * LTKV_BLOCK), part);
-  const int split =
-      short_rem ? 1 : ltkv::attention_split((int)c->elem, (int)group, (int)(c->kv_dim / P.head_dim));
-  const size_t max_parts = (size_t)parts * split;
-  if ((uint64_t)P.n * (P.n_heads / group) * max_parts * 256 >= (1ull << 32))
-    return fail(LTKV_ERR_ARG, "attention grid too large for one launch");
+  const PlanShape L = plan_shape(c);
+  if (L.too_large) return fail(LTKV_ERR_ARG, "attention grid too large for one launch");
+  const int part = L.part, split = L.split;
+  const size_t max_parts = L.max_parts, pre_o_off = L.pre_o_off, pre_ml_off = L.pre_ml_off;
 
   DeviceGuard dg(c->device);
   if (!dg.ok) return fail(LTKV_ERR_HIP, "hipSetDevice(%d) failed", c->device);
-  // (no partition partials where the groups cover every query's context)
-  ltkv::AttnWorkspace ws = ltkv::attention_workspace(
-      (int64_t)P.n, (int)P.n_heads, (int)P.head_dim, (int)max_parts, grouped && !P.pass_empty && !P.groups_only);
-  if (grouped && (P.pass_empty || P.groups_only)) ws = ltkv::AttnWorkspace{0, 0, 0};
-  const size_t pre_slots = grouped ? P.n * P.n_heads * (size_t)P.max_pre_parts : 0;
-  const size_t pre_o_off = ((size_t)ws.bytes + 255) / 256 * 256;
-  const size_t pre_ml_off = pre_o_off + pre_slots * P.head_dim * 4;
   uint8_t *base = nullptr;
-  const size_t ws_bytes = pre_ml_off + pre_slots * 2 * 4;
-  if (int rc = workspace(c, ws_bytes, &base)) return rc;
-  const size_t held_used = base == c->held ? ws_bytes : 0;
+  if (int rc = workspace(c, L.bytes, &base)) return rc;
+  const size_t held_used = base == c->held ? L.bytes : 0;
   const int32_t *d = reinterpret_cast<const int32_t *>(P.d);
   const ltkv::PoolGeom g = head_geom(c, P.head_dim);
-  ltkv::AttnArgs a = attn_args(c, layer, P.n, P.n_heads, P.head_dim, scale, d_q, d_out, ws, part,
+  ltkv::AttnArgs a = attn_args(c, layer, P.n, P.n_heads, P.head_dim, scale, d_q, d_out, L.ws, part,
                                (int)max_parts, base);
   a.split = split;
   set_wide_parts(c, a, group, P.sstride * LTKV_BLOCK, false);

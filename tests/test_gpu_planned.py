@@ -399,3 +399,35 @@ def test_merge_of_range_partials(gpu, n_heads, n_kv, head_dim, tokens):
     g, o, seqs, lens = _prefill_state(rng, n_kv * head_dim, [(0, tokens - 20, 20)])
     stats, *_ = _run(gpu, g, o, seqs, lens, n_heads, head_dim, rng)
     assert stats["groups"] == 1 and stats["grouped"] == 20
+
+
+def test_first_planned_attention_captured(gpu):
+    """A plan whose partials exceed what a cache holds from its creation (300
+    rows after 1400 tokens cut into ranges, beside two decodes): its first
+    attention call is a captured one, and the replays equal eager calls."""
+    import torch
+
+    from langtrain_studio_amd import KvCache
+
+    rng = np.random.default_rng(31)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        g = KvCache(1, 1024, 6000, dtype="f16", device=0, stream=stream)
+        fill_sequences([("gpu", g)], {0: 1700, 1: 1500, 2: 900}, rng, 1024)
+        seqs = np.array([0] * 300 + [1, 2], np.uint32)
+        lens = np.array(list(range(1401, 1701)) + [1500, 900], np.uint32)
+        g.plan_attention(seqs, lens, 32, 128, shared_prefix=True)
+        assert g.plan_stats()["grouped"] == 300
+        q = torch.randn((302, 32 * 128), device=gpu)
+        out = torch.zeros_like(q)
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            g.planned_attention(0, q, out=out)
+        for _ in range(3):
+            q.normal_()
+            graph.replay()
+            got = out.clone()
+            want = g.planned_attention(0, q)
+            stream.synchronize()
+            assert torch.equal(got.view(torch.int32), want.view(torch.int32))
