@@ -79,6 +79,7 @@ struct AttnPlan {
   size_t n_pass = 0;         // queries of the per-query pass (the rest are completed by groups)
   size_t n_plain = 0;        // ... of which the first n_plain of the query map have no group partials
   bool separate = false;     // ... and the others nothing but group partials: two launches
+  size_t n_busy = 0;         // ... and those with a remainder
   size_t max_suffix = 0;     // longest remainder (tokens) of a per-query-pass query
   bool empty_with_groups = false;  // a query with group partials and no remainder
   bool pass_empty = false;         // every per-query-pass query is such a query
@@ -944,7 +945,7 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
   if ((uint64_t)n * sstride + (uint64_t)groups.size() * gstride > (uint64_t)INT32_MAX / 2)
     return fail(LTKV_ERR_ARG, "block tables of this batch are too large");
   std::vector<int32_t> qmap;  // queries left for the per-query pass
-  size_t max_suffix = 0;
+  size_t max_suffix = 0, n_busy = 0;
   bool empty_with_groups = false, pass_empty = true, separate = true;
   // Queries without group partials first, then those with some.
   for (size_t i = 0; i < n; ++i)
@@ -959,6 +960,7 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
     if (pre_parts[i] >= 0) {
       const size_t rem = lens[i] > pre_tokens[i] ? lens[i] - pre_tokens[i] : 0;
       max_suffix = std::max(max_suffix, rem);
+      n_busy += rem > 0;
       if (pre_parts[i] > 0 && rem == 0) empty_with_groups = true;
       if (pre_parts[i] == 0 || rem > 0) pass_empty = false;
     }
@@ -979,6 +981,7 @@ int build_plan(ltkv_cache *c, size_t n, const uint32_t *seqs, const uint32_t *le
   P.n_plain = n_plain;
   P.separate = separate && n_plain > 0;
   P.max_suffix = max_suffix;
+  P.n_busy = n_busy;
   P.empty_with_groups = empty_with_groups;
   P.pass_empty = pass_empty && !groups_only;
   P.off_tables = 0;
@@ -1891,6 +1894,7 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
   // decode kernel writes every output itself (folding group partials).
   a.merge_free = grouped && part > 0 && P.max_suffix <= (size_t)(part / split) && !P.empty_with_groups;
   a.short_rest = grouped && P.max_suffix <= kShortRemainder;
+  a.busy = (int64_t)P.n_busy;
   a.pass_empty = grouped && P.pass_empty;
   a.tables = d + P.off_stables;
   a.table_stride = (int64_t)P.sstride;
@@ -1949,14 +1953,26 @@ int ltkv_planned_attention(ltkv_cache *c, size_t layer, float scale, const float
     w.n = (int64_t)P.n_plain;
     w.qmap = d + P.off_qmap;
     w.pre_parts = nullptr;
-    w.merge_free = w.short_rest = false;
-    set_subs(w);
-    HIP_TRY(ltkv::launch_decode_attention(g, w, c->stream), "decode attention launch");
-    if (P.n_pass == P.n_plain) return LTKV_OK;
-    a.n = (int64_t)(P.n_pass - P.n_plain);
-    a.qmap = d + P.off_qmap + P.n_plain;
-    a.merge_free = false;
-    a.pass_empty = true;
+    // Each in one partition no longer than a part: nothing to merge. Partitions
+    // of 64 tokens or less at head_dim 64 gain nothing from waves of their own
+    // (17 decodes of 57-241 tokens, TinyLlama 29.6 us without, 30.1-30.6 with;
+    // Llama-3-8B 35.3 / 33.3; 32 of 2-40 tokens 24.7 / 26.5).
+    w.merge_free = part > 0 && P.max_suffix <= (size_t)(part / split) &&
+                   P.max_suffix <= (size_t)ltkv::sub_tokens(0, (int)P.head_dim);
+    if (!w.merge_free && (part <= 0 || (size_t)(part / split) * P.head_dim > 4096)) set_subs(w);
+    // One pass where the launch more is not made up for: short decodes too many
+    // for a wave per part, and few chunk rows beside them (60 decodes of 300-500
+    // tokens and 72 rows, TinyLlama: 39.9 us in one pass, 42.0 in two; 20 and
+    // 40 rows, Llama-3-8B, 48.6 / 48.8; 20 and 400 rows 75.8 / 58.2).
+    const size_t rest = P.n_pass - P.n_plain;
+    if (w.merge_free || w.subs > 0 || !a.short_rest || rest == 0 || rest > 2 * P.n_plain) {
+      HIP_TRY(ltkv::launch_decode_attention(g, w, c->stream), "decode attention launch");
+      if (rest == 0) return LTKV_OK;
+      a.n = (int64_t)rest;
+      a.qmap = d + P.off_qmap + P.n_plain;
+      a.merge_free = false;
+      a.pass_empty = true;
+    }
   }
   HIP_TRY(ltkv::launch_decode_attention(g, a, c->stream), "decode attention launch");
   return LTKV_OK;

@@ -135,8 +135,9 @@ struct AttnArgs {
   // matrix-core kernel folds group partials of single-partition queries).
   bool merge_free;
   // The caller knows that every query reads a short remainder after group
-  // partials (decode_ordered).
+  // partials, `busy` of them any at all (decode_ordered).
   bool short_rest;
+  int64_t busy;
   // The caller knows the context kernel has nothing to do: every query has
   // group partials and an empty remainder, so only the merge runs (it folds
   // the group partials by itself).

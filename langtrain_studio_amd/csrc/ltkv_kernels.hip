@@ -2980,14 +2980,15 @@ attn_mfma_kernel(const T *__restrict__ kpool, const T *__restrict__ vpool, const
 // (Qwen2.5-7B, one query map entry each) 233 us in query order, 162 us so.
 // Short remainders after group partials (short_rest) are nearly equal and pay
 // each wave's scan for little: in one partition each they keep query order,
-// and otherwise as long as all waves start at once (four a CU). Forks of 992
+// and otherwise as long as all waves with something to read start at once
+// (four a CU). Forks of 992
 // shared tokens, Llama-3-8B f16, us a step, query order / longest first: 5 of
 // 138 own tokens 26.4 / 27.1, 32 32.1 / 32.8, 128 (1024 waves) 50.9 / 50.1,
 // 128 of 488 73.9 / 75.5; 200 of 138 (1600 waves) 70.0 / 65.1, 200 of 488
 // 123.6 / 110.1.
 inline bool decode_ordered(const AttnArgs &a, int64_t waves) {
   if (a.merge_free || a.n <= 1 || a.n > kOrderMaxQueries) return false;
-  return !a.short_rest || waves > 4 * (int64_t)a.cu_count;
+  return !a.short_rest || waves / a.n * a.busy > 4 * (int64_t)a.cu_count;
 }
 
 // One wave per item (a partition of NH kv heads of one query), kDecodeWaves

@@ -431,3 +431,23 @@ def test_first_planned_attention_captured(gpu):
             want = g.planned_attention(0, q)
             stream.synchronize()
             assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("n_heads,n_kv,head_dim,chunk,ctx,decodes", [
+    (32, 8, 128, 24, 30, (2, 41, 9)),       # one partition and part each: no merge
+    (32, 4, 64, 24, 30, (64, 300, 40)),     # at most a part each, some of two partitions
+    (32, 4, 64, 24, 120, (57, 242, 17)),    # 64-token partitions at head_dim 64
+    (32, 8, 128, 24, 120, (57, 242, 17)),
+    (32, 4, 64, 24, 500, (300, 501, 60)),   # cut ranges and the decodes in one pass
+    (32, 4, 64, 200, 500, (300, 501, 60)),  # ... in two
+])
+def test_short_decodes_beside_chunks(gpu, n_heads, n_kv, head_dim, chunk, ctx, decodes):
+    """Decodes of up to 512 tokens beside three prompt chunks: the forms their
+    pass takes by the partitions' length and the chunk rows beside them."""
+    rng = np.random.default_rng(chunk + ctx + decodes[2])
+    lo, hi, n = decodes
+    lens = [hi - 1, lo] + [int(x) for x in rng.integers(lo, hi, n - 2)]
+    g, o, seqs, lens = _prefill_state(rng, n_kv * head_dim, [(s, ctx + s, chunk) for s in range(3)],
+                                      decode=[(10 + i, x) for i, x in enumerate(lens)])
+    stats, *_ = _run(gpu, g, o, seqs, lens, n_heads, head_dim, rng)
+    assert stats["groups"] == 3 and stats["grouped"] == 3 * chunk
